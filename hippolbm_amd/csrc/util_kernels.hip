@@ -306,75 +306,72 @@ __global__ void k_macro(const void* fv, uint64_t stride, uint32_t N, const uint8
 }
 
 // simulation_state (simulation_state.hpp:47-79): per-block partial sums in
-// FP64, then one block folds the partials in a fixed order (deterministic).
+// FP64, then one block folds the partials, both in a fixed order
+// (deterministic).  Seven values per record: sum rho, min |u|, max |u|, the
+// three sums of rho u, the number of fluid nodes.
 constexpr int RED_BLOCK = 256;
+constexpr int RED_VALUES = 7;
+
+__device__ __forceinline__ double red_combine(int k, double a, double b) {
+  return k == 1 ? fmin(a, b) : (k == 2 ? fmax(a, b) : a + b);
+}
+
+// Folds every thread's record of the block into thread 0's (and writes it to out).
+__device__ __forceinline__ void red_block(double (&v)[RED_VALUES], double* out) {
+  __shared__ double s[RED_VALUES][RED_BLOCK];
+  const int t = threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < RED_VALUES; k++) s[k][t] = v[k];
+  __syncthreads();
+  for (int w = RED_BLOCK / 2; w > 0; w >>= 1) {
+    if (t < w) {
+#pragma unroll
+      for (int k = 0; k < RED_VALUES; k++) s[k][t] = red_combine(k, s[k][t], s[k][t + w]);
+    }
+    __syncthreads();
+  }
+  if (t < RED_VALUES) out[t] = s[t][0];
+}
+
+__device__ __forceinline__ void red_init(double (&v)[RED_VALUES]) {
+#pragma unroll
+  for (int k = 0; k < RED_VALUES; k++) v[k] = k == 1 ? 1.7976931348623157e308 : (k == 2 ? -1.7976931348623157e308 : 0.0);
+}
 
 __global__ void __launch_bounds__(RED_BLOCK)
     k_reduce_partial(const double* m0, const double* m1, const uint8_t* flags, uint32_t N, double* part) {
-  __shared__ double s_sum[RED_BLOCK], s_min[RED_BLOCK], s_max[RED_BLOCK], s_jx[RED_BLOCK], s_jy[RED_BLOCK],
-      s_jz[RED_BLOCK], s_cnt[RED_BLOCK];
-  double sum = 0.0, vmin = 1.7976931348623157e308, vmax = -1.7976931348623157e308, jx = 0.0, jy = 0.0, jz = 0.0,
-         cnt = 0.0;
+  double v[RED_VALUES];
+  red_init(v);
   const uint32_t stride = gridDim.x * RED_BLOCK;
   for (uint32_t i = blockIdx.x * RED_BLOCK + threadIdx.x; i < N; i += stride) {
     const double r = m0[i];
     const double ux = m1[i], uy = m1[(size_t)N + i], uz = m1[2 * (size_t)N + i];
-    const double v = sqrt(ux * ux + uy * uy + uz * uz);
-    sum += r;
-    vmin = fmin(vmin, v);
-    vmax = fmax(vmax, v);
-    jx += r * ux;
-    jy += r * uy;
-    jz += r * uz;
-    cnt += flags[i] ? 0.0 : 1.0;
+    const double n = sqrt(ux * ux + uy * uy + uz * uz);
+    v[0] += r;
+    v[1] = fmin(v[1], n);
+    v[2] = fmax(v[2], n);
+    v[3] += r * ux;
+    v[4] += r * uy;
+    v[5] += r * uz;
+    v[6] += flags[i] ? 0.0 : 1.0;
   }
-  const int t = threadIdx.x;
-  s_sum[t] = sum;
-  s_min[t] = vmin;
-  s_max[t] = vmax;
-  s_jx[t] = jx;
-  s_jy[t] = jy;
-  s_jz[t] = jz;
-  s_cnt[t] = cnt;
-  __syncthreads();
-  for (int w = RED_BLOCK / 2; w > 0; w >>= 1) {
-    if (t < w) {
-      s_sum[t] += s_sum[t + w];
-      s_min[t] = fmin(s_min[t], s_min[t + w]);
-      s_max[t] = fmax(s_max[t], s_max[t + w]);
-      s_jx[t] += s_jx[t + w];
-      s_jy[t] += s_jy[t + w];
-      s_jz[t] += s_jz[t + w];
-      s_cnt[t] += s_cnt[t + w];
-    }
-    __syncthreads();
-  }
-  if (t == 0) {
-    double* o = part + 7 * (size_t)blockIdx.x;
-    o[0] = s_sum[0];
-    o[1] = s_min[0];
-    o[2] = s_max[0];
-    o[3] = s_jx[0];
-    o[4] = s_jy[0];
-    o[5] = s_jz[0];
-    o[6] = s_cnt[0];
-  }
+  red_block(v, part + RED_VALUES * (size_t)blockIdx.x);
 }
 
-__global__ void k_reduce_final(const double* part, int nparts, double* out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  double r[7] = {0.0, 1.7976931348623157e308, -1.7976931348623157e308, 0.0, 0.0, 0.0, 0.0};
-  for (int b = 0; b < nparts; b++) {
-    const double* o = part + 7 * (size_t)b;
-    r[0] += o[0];
-    r[1] = fmin(r[1], o[1]);
-    r[2] = fmax(r[2], o[2]);
-    r[3] += o[3];
-    r[4] += o[4];
-    r[5] += o[5];
-    r[6] += o[6];
+// The up to 1024 partials are latency-bound: one thread walking them alone made
+// a chain of dependent loads (20 us for the 117 partials of a 31^3 grid, about
+// 220 us for 1024); a block of 256 threads takes at most four records each and
+// then the same tree as the partial kernel: hlbm_reduce_stats 257 -> 27 us at
+// 64^3, a step with its log line at 31^3 53 -> 28 us.
+__global__ void __launch_bounds__(RED_BLOCK) k_reduce_final(const double* part, int nparts, double* out) {
+  double v[RED_VALUES];
+  red_init(v);
+  for (int b = threadIdx.x; b < nparts; b += RED_BLOCK) {
+    const double* o = part + RED_VALUES * (size_t)b;
+#pragma unroll
+    for (int k = 0; k < RED_VALUES; k++) v[k] = red_combine(k, v[k], o[k]);
   }
-  for (int k = 0; k < 7; k++) out[k] = r[k];
+  red_block(v, out);
 }
 
 // plane_velocity_profile (src/check/plane_velocity_profile.cu:81-101): per
@@ -813,7 +810,7 @@ hipError_t launch_reduce(const double* m0, const double* m1, const uint8_t* flag
   hipLaunchKernelGGL(k_reduce_partial, dim3(parts), dim3(RED_BLOCK), 0, s, m0, m1, flags, N, part);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(64), 0, s, (const double*)part, parts, out);
+  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(RED_BLOCK), 0, s, (const double*)part, parts, out);
   return hipGetLastError();
 }
 
