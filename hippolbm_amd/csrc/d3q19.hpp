@@ -99,6 +99,24 @@ HLBM_HD inline uint32_t node_at(const NodeLayout& L, int x, int y, int z) {
   return (uint32_t)x * L.st[0] + (uint32_t)y * L.st[1] + (uint32_t)z * L.st[2];
 }
 
+// Division of node indices by a row length (n0) and a plane size (n0 * n1) as
+// one 32-bit multiply-high and a shift each: with s = ceil(log2 d) and
+// m = floor(2^(31+s) / d) + 1, floor(n / d) = (n m) >> (31 + s) for every
+// n < 2^31, since n (m d - 2^(31+s)) <= n d < 2^(31+s).  2 <= d < 2^31.
+struct NodeDivisors {
+  uint32_t m0, s0;    // row length
+  uint32_t m01, s01;  // plane size
+};
+inline void node_divisor(uint32_t d, uint32_t& m, uint32_t& s) {
+  uint32_t l = 0;
+  while ((1ull << l) < d) l++;
+  m = (uint32_t)((1ull << (31 + l)) / d + 1);
+  s = l - 1;
+}
+HLBM_HD inline uint32_t div_by(uint32_t n, uint32_t m, uint32_t s) {
+  return (uint32_t)(((uint64_t)n * m) >> 32) >> s;
+}
+
 // plane index (hlbm_plane) -> (dim, side)
 HLBM_HD constexpr int plane_dim(int p) { return p < 2 ? 2 : (p < 4 ? 1 : 0); }
 HLBM_HD constexpr int plane_side(int p) { return p & 1; }

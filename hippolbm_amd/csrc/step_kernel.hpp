@@ -75,7 +75,7 @@ struct StepParams {
   int32_t nx, ny, nz;
   int32_t per[3];
   uint32_t N;           // nodes
-  uint32_t pad0;
+  int32_t linear;       // bulk kernel: consecutive nodes per workgroup instead of tiles (NodeDivisors set)
   uint64_t stride;      // elements between two population planes
   NodeLayout lay;       // node (x, y, z) at lay.st . (x, y, z); lay.ord: the axes, fastest first
   int32_t ln[3];        // nodes along lay.ord[0..2] (the bulk kernel's lane, row and grid axes)
@@ -128,6 +128,7 @@ struct StepParams {
   int32_t set_box[MAX_SET][6]; // node box, inclusive: x0 y0 z0 x1 y1 z1
   double set_val[MAX_SET];     // f_i = value * w_i
   float mrtf[10];              // the MRT rates in FP32 (defaults or custom), for the FP32-compute forms
+  NodeDivisors div;            // the layout's row and plane sizes as divisors (linear)
 };
 
 // ---------------------------------------------------------------------------
@@ -1329,14 +1330,52 @@ __global__ void __launch_bounds__(256) step_kernel(const StepParams p) {
     const uint32_t per = nt / 8u;
     if (t < per * 8u) t = (t % 8u) * per + t / 8u;
   }
-  // lanes run along the layout's fastest axis, tile rows along the next one and
-  // the grid along the slowest: l, row and c2 below
-  const int bx = (int)(t % (uint32_t)p.gx);
-  const uint32_t r = t / (uint32_t)p.gx;
-  const int by = (int)(r % (uint32_t)p.gy);
-  const int c2 = (int)(r / (uint32_t)p.gy);
-  const int l = bx * blockDim.x + threadIdx.x;
-  if (l >= p.ln[0] || c2 >= p.ln[2]) return;
+  // lanes run along the layout's fastest axis, rows along the next one and the
+  // grid along the slowest: l, row0 and c2 below
+  int l, row0, c2;
+  uint32_t n = 0;
+  const bool linear = NPT == 1 && p.linear;
+  if (linear) {
+    // Consecutive nodes per workgroup: every lane works and every wave's rows
+    // of populations start on a cache line, whatever the row length.  The
+    // wave's first node is divided in scalar registers; rows of 64 nodes and
+    // more then hold at most one row end per wave.
+    const uint32_t tid = threadIdx.y * blockDim.x + threadIdx.x;
+    const uint32_t first =
+        t * (blockDim.x * blockDim.y) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid & ~63u));
+    const uint32_t n0 = (uint32_t)p.ln[0], n1 = (uint32_t)p.ln[1], n01 = n0 * n1;
+    n = first + (tid & 63u);
+    if (n >= p.N) return;
+    if (n0 >= 64u) {
+      const uint32_t k2 = div_by(first, p.div.m01, p.div.s01), r = first - k2 * n01;
+      const uint32_t k1 = div_by(r, p.div.m0, p.div.s0);
+      l = (int)(r - k1 * n0 + (tid & 63u));
+      row0 = (int)k1;
+      c2 = (int)k2;
+      if (l >= (int)n0) {
+        l -= (int)n0;
+        row0++;
+        if (row0 == (int)n1) {
+          row0 = 0;
+          c2++;
+        }
+      }
+    } else {
+      const uint32_t k2 = div_by(n, p.div.m01, p.div.s01), r = n - k2 * n01;
+      const uint32_t k1 = div_by(r, p.div.m0, p.div.s0);
+      l = (int)(r - k1 * n0);
+      row0 = (int)k1;
+      c2 = (int)k2;
+    }
+  } else {
+    const int bx = (int)(t % (uint32_t)p.gx);
+    const uint32_t r = t / (uint32_t)p.gx;
+    const int by = (int)(r % (uint32_t)p.gy);
+    c2 = (int)(r / (uint32_t)p.gy);
+    l = bx * blockDim.x + threadIdx.x;
+    row0 = by * NPT * blockDim.y + threadIdx.y;
+    if (l >= p.ln[0] || c2 >= p.ln[2]) return;
+  }
   const int o0 = PERM ? p.lay.ord[0] : 0, o1 = PERM ? p.lay.ord[1] : 1;
   auto coords = [&](int row, int& x, int& y, int& z) {
     if constexpr (PERM) {
@@ -1351,6 +1390,7 @@ __global__ void __launch_bounds__(256) step_kernel(const StepParams p) {
   };
   // the default layout: the node index and the stochastic-rounding key coincide
   auto index_of = [&](int x, int y, int z) -> uint32_t {
+    if (linear) return n;
     if constexpr (PERM)
       return node_index(p, x, y, z);
     else
@@ -1363,7 +1403,7 @@ __global__ void __launch_bounds__(256) step_kernel(const StepParams p) {
     bool wall[NPT], act[NPT];
 #pragma unroll
     for (int k = 0; k < NPT; k++) {
-      const int row = (by * NPT + k) * blockDim.y + threadIdx.y;
+      const int row = row0 + k * (int)blockDim.y;
       int x, y, z;
       coords(row, x, y, z);
       act[k] = row < p.ln[1] && !(MODE != MODE_COLLIDE && (node_planes(x, y, z, p.nx, p.ny, p.nz) & p.prog_planes));
@@ -1402,7 +1442,7 @@ __global__ void __launch_bounds__(256) step_kernel(const StepParams p) {
   bool wall[NPT], act[NPT];
 #pragma unroll
   for (int k = 0; k < NPT; k++) {
-    const int row = (by * NPT + k) * blockDim.y + threadIdx.y;
+    const int row = row0 + k * (int)blockDim.y;
     int& x = xs[k];
     int& y = ys[k];
     int& z = zs[k];
