@@ -19,6 +19,7 @@
 #include "../../include/hlbm.h"
 #include "common.hpp"
 #include "launch.hpp"
+#include "transfer.hpp"
 #include "util_kernels.hpp"
 
 using namespace hlbm;
@@ -885,8 +886,32 @@ static int ensure_tmp(hlbm_domain* h) {
   return HLBM_OK;
 }
 
+static TransferGrid transfer_grid(const hlbm_domain* h, int32_t layout) {
+  return TransferGrid{{h->nx, h->ny, h->nz}, h->lay, layout == HLBM_LAYOUT_REF, h->d.storage, dom_shift(h)};
+}
+
+// The 19 population planes of the current buffer and a host array of them.
+static std::array<NodePlane, Q> population_planes(hlbm_domain* h, const double* f, int32_t layout) {
+  const size_t per = layout == HLBM_LAYOUT_REF ? ref_count(h) : (size_t)h->N;
+  std::array<NodePlane, Q> p;
+  for (int i = 0; i < Q; i++)
+    p[i] = NodePlane{(char*)h->buf[h->cur] + (size_t)i * h->stride * h->esize, const_cast<double*>(f) + i * per, i};
+  return p;
+}
+
 int hlbm_set_populations_f64(hlbm_domain* h, const double* f, int32_t layout) {
   if (!h || !f) return fail(HLBM_ERR_ARG, "NULL argument");
+  {
+    const auto planes = population_planes(h, f, layout);
+    hipError_t e = hipSuccess;
+    const int t = planes_to_device(transfer_grid(h, layout), planes.data(), Q, 0, &e);
+    if (t == TRANSFER_FAILED) return fail(HLBM_ERR_HIP, std::string("populations in: ") + hipGetErrorString(e));
+    if (t == TRANSFER_DONE) {
+      HIP_TRY(hipDeviceSynchronize());
+      h->phase = PHASE_PRE;
+      return HLBM_OK;
+    }
+  }
   int rc = ensure_tmp(h);
   if (rc) return rc;
   std::vector<double> plane, lplane;
@@ -969,6 +994,16 @@ int hlbm_get_populations_f64(hlbm_domain* h, double* f, int32_t layout) {
   if (!h || !f) return fail(HLBM_ERR_ARG, "NULL argument");
   int rc = materialize(h, 0);
   if (rc) return rc;
+  {
+    const auto planes = population_planes(h, f, layout);
+    hipError_t e = hipSuccess;
+    const int t = planes_to_host(transfer_grid(h, layout), planes.data(), Q, 0, &e);
+    if (t == TRANSFER_FAILED) return fail(HLBM_ERR_HIP, std::string("populations out: ") + hipGetErrorString(e));
+    if (t == TRANSFER_DONE) {
+      if (layout == HLBM_LAYOUT_REF) fill_periodic_ghosts(h, f, Q);
+      return HLBM_OK;
+    }
+  }
   rc = ensure_tmp(h);
   if (rc) return rc;
   std::vector<double> plane(layout == HLBM_LAYOUT_REF ? h->N : 0), lplane(default_layout_p(h) ? 0 : h->N);
@@ -1040,6 +1075,22 @@ int hlbm_synchronize(hlbm_domain* h) {
 
 static int copy_macro_out(hlbm_domain* h, double* rho, double* u, int32_t layout) {
   const size_t N = h->N;
+  {
+    NodePlane p[4];
+    int n = 0;
+    if (rho) p[n++] = NodePlane{h->m0, rho, -1};
+    for (int c = 0; u && c < 3; c++)
+      p[n++] = NodePlane{h->m1 + c * N, u + c * (layout == HLBM_LAYOUT_REF ? ref_count(h) : N), -1};
+    hipError_t e = hipSuccess;
+    const int t = planes_to_host(transfer_grid(h, layout), p, n, 0, &e);
+    if (t == TRANSFER_FAILED) return fail(HLBM_ERR_HIP, std::string("rho and u out: ") + hipGetErrorString(e));
+    if (t == TRANSFER_DONE) return HLBM_OK;
+  }
+  if (layout != HLBM_LAYOUT_REF && default_layout_p(h)) {
+    if (rho) HIP_TRY(hipMemcpy(rho, h->m0, N * 8, hipMemcpyDeviceToHost));
+    if (u) HIP_TRY(hipMemcpy(u, h->m1, 3 * N * 8, hipMemcpyDeviceToHost));
+    return HLBM_OK;
+  }
   std::vector<double> r(N), v(3 * N);
   HIP_TRY(hipMemcpy(r.data(), h->m0, N * 8, hipMemcpyDeviceToHost));
   HIP_TRY(hipMemcpy(v.data(), h->m1, 3 * N * 8, hipMemcpyDeviceToHost));

@@ -1,0 +1,315 @@
+// transfer.hip -- FP64 per-node arrays between HBM and pageable host memory.
+//
+// Compiled with -ffp-contract=off (the shift arithmetic rounds as the plain
+// conversion kernels' does).
+//
+// A host array that a program has just allocated is bound by its page faults
+// (one thread writes 4.8 GB/s into fresh pages, eight 26-38 GB/s), and a copy
+// into pageable memory through the runtime reaches 4 GB/s.  So a call takes a
+// ring of pinned slots, kernels move the data between HBM and the slots in node
+// order at the link's rate (53 GB/s to the host, 55 from it; conversion and
+// layout cost nothing there), and a few threads move it between the slots and
+// the caller's array, both sides running ahead of each other by half a ring.
+// Measured against copies plane by plane through the runtime: 400 steps of the
+// porous channel 256 x 128 x 128 (layout "yzx") with rho and u read 215 -> 105
+// ms, 300 MRT steps of 128^3 FP32 35.5 -> 20.2 ms, populations of 96^3 in and
+// out 18.5 -> 9.3 ms.
+//
+// The slots and threads live as long as the call (a pinned allocation of this
+// size costs about 20 us once the process has had one).
+#include <algorithm>
+#include <condition_variable>
+#include <cstring>
+#include <functional>
+#include <mutex>
+#include <new>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+#include "step_kernel.hpp"
+#include "transfer.hpp"
+
+namespace hlbm {
+namespace {
+
+// Smaller transfers gain nothing over the runtime's own copies.
+constexpr size_t TRANSFER_MIN_BYTES = (size_t)4 << 20;
+constexpr size_t SLOT_MAX = (size_t)1 << 20, SLOT_MIN = (size_t)256 << 10;
+constexpr int SLOTS = 16, THREADS = 8;
+
+// node k of the host's order (x fastest) -> index in the device layout
+struct NodeOrder {
+  uint32_t nx, nxy;
+  NodeDivisors div;
+  NodeLayout lay;
+};
+template <bool PERM>
+__device__ __forceinline__ uint32_t device_index(const NodeOrder& o, uint32_t k) {
+  if constexpr (!PERM) {
+    return k;
+  } else {
+    const uint32_t z = div_by(k, o.div.m01, o.div.s01), r = k - z * o.nxy;
+    const uint32_t y = div_by(r, o.div.m0, o.div.s0);
+    return node_at(o.lay, (int)(r - y * o.nx), (int)y, (int)z);
+  }
+}
+
+// nodes [first, first + n) between a device plane and a slot; w + sig is the
+// rest state of the plane's direction
+template <class S, bool PERM>
+__global__ void __launch_bounds__(256) k_export(const S* src, double* slot, uint32_t first, uint32_t n, NodeOrder o,
+                                                double w, double sig) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t j = device_index<PERM>(o, first + i);
+  if constexpr (StoreOps<S>::shifted)
+    slot[i] = (double)StoreOps<S>::ld(src, j) + (w + sig);
+  else
+    slot[i] = src[j];
+}
+template <class S, bool PERM>
+__global__ void __launch_bounds__(256) k_import(S* dst, const double* slot, uint32_t first, uint32_t n, NodeOrder o,
+                                                double w, double sig) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t j = device_index<PERM>(o, first + i);
+  if constexpr (StoreOps<S>::shifted)
+    StoreOps<S>::st(dst, j, (float)(slot[i] - w - sig));
+  else
+    dst[j] = slot[i];
+}
+
+template <class S>
+hipError_t move_t(bool out, void* dev, double* slot, uint32_t first, uint32_t n, const NodeOrder& o, bool perm,
+                  double w, double sig, hipStream_t s) {
+  const dim3 g((n + 255) / 256), b(256);
+  if (out) {
+    if (perm)
+      hipLaunchKernelGGL((k_export<S, true>), g, b, 0, s, (const S*)dev, slot, first, n, o, w, sig);
+    else
+      hipLaunchKernelGGL((k_export<S, false>), g, b, 0, s, (const S*)dev, slot, first, n, o, w, sig);
+  } else {
+    if (perm)
+      hipLaunchKernelGGL((k_import<S, true>), g, b, 0, s, (S*)dev, (const double*)slot, first, n, o, w, sig);
+    else
+      hipLaunchKernelGGL((k_import<S, false>), g, b, 0, s, (S*)dev, (const double*)slot, first, n, o, w, sig);
+  }
+  return hipGetLastError();
+}
+
+// Host side of a chunk: nodes [first, first + n) between the slot and a plane.
+void copy_rows(const TransferGrid& g, bool out, double* slot, double* host, uint32_t first, uint32_t n) {
+  if (!g.reference) {
+    if (out)
+      std::memcpy(host + first, slot, (size_t)n * 8);
+    else
+      std::memcpy(slot, host + first, (size_t)n * 8);
+    return;
+  }
+  // the All box: two ghost layers per side
+  const uint32_t nx = (uint32_t)g.n[0], ny = (uint32_t)g.n[1];
+  const size_t Lx = nx + 4, Ly = ny + 4;
+  for (uint32_t k = first; k < first + n;) {
+    const uint32_t row = k / nx, x = k - row * nx, z = row / ny, y = row - z * ny;
+    const uint32_t len = std::min(nx - x, first + n - k);
+    double* h = host + ((size_t)(z + 2) * Ly + (y + 2)) * Lx + (x + 2);
+    double* p = slot + (k - first);
+    if (out)
+      std::memcpy(h, p, (size_t)len * 8);
+    else
+      std::memcpy(p, h, (size_t)len * 8);
+    k += len;
+  }
+}
+
+struct Chunk {
+  int plane;
+  uint32_t first, n;
+};
+
+// Host-side copies of chunks 0, 1, 2, ..., done by a few threads as they are released.
+class Copiers {
+ public:
+  template <class F>
+  Copiers(int chunks, F&& job) : done_(chunks, 0), job_(std::forward<F>(job)) {}
+  // false if not one thread could be started
+  bool start(int threads) {
+    try {
+      for (int k = 0; k < threads; k++) pool_.emplace_back([this] { work(); });
+    } catch (const std::system_error&) {
+    }
+    return !pool_.empty();
+  }
+  ~Copiers() {
+    {
+      std::lock_guard<std::mutex> l(mu_);
+      stop_ = true;
+    }
+    todo_cv_.notify_all();
+    for (auto& t : pool_) t.join();
+  }
+  // the next chunk may be copied
+  void release_next() {
+    {
+      std::lock_guard<std::mutex> l(mu_);
+      released_++;
+    }
+    todo_cv_.notify_one();
+  }
+  void wait(int c) {
+    std::unique_lock<std::mutex> l(mu_);
+    done_cv_.wait(l, [&] { return done_[c] != 0; });
+  }
+
+ private:
+  void work() {
+    for (;;) {
+      int c;
+      {
+        std::unique_lock<std::mutex> l(mu_);
+        todo_cv_.wait(l, [&] { return stop_ || taken_ < released_; });
+        if (taken_ == released_) return;
+        c = taken_++;
+      }
+      job_(c);
+      {
+        std::lock_guard<std::mutex> l(mu_);
+        done_[c] = 1;
+      }
+      done_cv_.notify_one();
+    }
+  }
+  std::mutex mu_;
+  std::condition_variable todo_cv_, done_cv_;
+  int released_ = 0, taken_ = 0;
+  std::vector<char> done_;
+  bool stop_ = false;
+  std::function<void(int)> job_;
+  std::vector<std::thread> pool_;
+};
+
+// The pinned ring and its events, given back on every way out.
+struct Ring {
+  double* mem = nullptr;
+  hipEvent_t ev[SLOTS] = {};
+  ~Ring() {
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (mem) (void)hipHostFree(mem);
+  }
+  bool open(size_t bytes, int slots) {
+    if (hipHostMalloc((void**)&mem, bytes * slots, hipHostMallocCoherent) != hipSuccess) {
+      mem = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+    for (int k = 0; k < slots; k++)
+      if (hipEventCreateWithFlags(&ev[k], hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
+        ev[k] = nullptr;
+        return false;
+      }
+    return true;
+  }
+};
+
+int transfer(bool out, const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s, hipError_t* err) {
+  *err = hipSuccess;
+  const uint32_t N = (uint32_t)g.n[0] * (uint32_t)g.n[1] * (uint32_t)g.n[2];
+  const size_t total = (size_t)N * 8 * count;
+  if (total < TRANSFER_MIN_BYTES) return TRANSFER_DECLINED;
+  const size_t slot_bytes = std::min(SLOT_MAX, std::max(SLOT_MIN, total / 32 / 4096 * 4096));
+  const uint32_t per = (uint32_t)(slot_bytes / 8);
+  std::vector<Chunk> chunks;
+  for (int p = 0; p < count; p++)
+    for (uint32_t a = 0; a < N; a += per) chunks.push_back({p, a, std::min(per, N - a)});
+  const int nc = (int)chunks.size(), slots = std::min(SLOTS, nc), ahead = slots / 2;
+  if (ahead < 1) return TRANSFER_DECLINED;
+
+  NodeOrder o;
+  o.nx = (uint32_t)g.n[0];
+  o.nxy = o.nx * (uint32_t)g.n[1];
+  node_divisor(o.nx, o.div.m0, o.div.s0);
+  node_divisor(o.nxy, o.div.m01, o.div.s01);
+  o.lay = g.lay;
+  const bool perm = !(g.lay.ord[0] == 0 && g.lay.ord[1] == 1);
+
+  Ring ring;
+  if (!ring.open(slot_bytes, slots)) return TRANSFER_DECLINED;
+  auto slot = [&](int c) { return ring.mem + (size_t)(c % slots) * per; };
+  Copiers copiers(nc, [&](int c) {
+    const Chunk& k = chunks[c];
+    copy_rows(g, out, slot(c), planes[k.plane].host, k.first, k.n);
+  });
+  if (!copiers.start(std::min(THREADS, nc))) return TRANSFER_DECLINED;
+
+  auto device = [&](int c) -> hipError_t {
+    const Chunk& k = chunks[c];
+    const NodePlane& p = planes[k.plane];
+    const double w = p.q < 0 ? 0.0 : WD(p.q), sig = p.q < 0 ? 0.0 : g.shift.s[dir_class(p.q)];
+    hipError_t e = hipErrorInvalidValue;
+    switch (p.q < 0 ? 0 : g.storage) {
+      case 0: e = move_t<double>(out, p.dev, slot(c), k.first, k.n, o, perm, w, sig, s); break;
+      case 1: e = move_t<float>(out, p.dev, slot(c), k.first, k.n, o, perm, w, sig, s); break;
+      case 2: e = move_t<_Float16>(out, p.dev, slot(c), k.first, k.n, o, perm, w, sig, s); break;
+      case 3: e = move_t<bf16s>(out, p.dev, slot(c), k.first, k.n, o, perm, w, sig, s); break;
+    }
+    return e == hipSuccess ? hipEventRecord(ring.ev[c % slots], s) : e;
+  };
+  auto landed = [&](int c) { return hipEventSynchronize(ring.ev[c % slots]); };
+
+  hipError_t e = hipSuccess;
+  if (out) {
+    // chunk c's kernel is queued when the chunk that held its slot has been
+    // copied out; chunk c - ahead is handed to the threads when it has landed
+    for (int c = 0; c < nc + ahead && e == hipSuccess; c++) {
+      if (c < nc) {
+        if (c >= slots) copiers.wait(c - slots);
+        e = device(c);
+      }
+      if (e == hipSuccess && c >= ahead) {
+        e = landed(c - ahead);
+        if (e == hipSuccess) copiers.release_next();
+      }
+    }
+    if (e == hipSuccess)
+      for (int c = std::max(0, nc - slots); c < nc; c++) copiers.wait(c);
+  } else {
+    // chunk c is filled when the kernel that read its slot has finished; chunk
+    // c - ahead's kernel is queued when it has been filled
+    for (int c = 0; c < nc + ahead && e == hipSuccess; c++) {
+      if (c < nc) {
+        if (c >= slots) e = landed(c - slots);
+        if (e == hipSuccess) copiers.release_next();
+      }
+      if (e == hipSuccess && c >= ahead) {
+        copiers.wait(c - ahead);
+        e = device(c - ahead);
+      }
+    }
+  }
+  // nothing may still read or write the slots when they are freed
+  const hipError_t last = hipStreamSynchronize(s);
+  *err = e != hipSuccess ? e : last;
+  return *err == hipSuccess ? TRANSFER_DONE : TRANSFER_FAILED;
+}
+
+int guarded(bool out, const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s, hipError_t* err) {
+  try {
+    return transfer(out, g, planes, count, s, err);
+  } catch (const std::bad_alloc&) {  // before any work: the lists and threads come first
+    *err = hipErrorOutOfMemory;
+    return TRANSFER_FAILED;
+  }
+}
+
+}  // namespace
+
+int planes_to_host(const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s, hipError_t* err) {
+  return guarded(true, g, planes, count, s, err);
+}
+int planes_to_device(const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s, hipError_t* err) {
+  return guarded(false, g, planes, count, s, err);
+}
+
+}  // namespace hlbm
