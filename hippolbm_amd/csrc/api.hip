@@ -38,6 +38,13 @@ namespace {
 // AA_SWAPPED (AA): post-collision populations in the opposite slots of each node.
 enum Phase { PHASE_PRE = 0, PHASE_POST = 1, PHASE_AA_PENDING = 2, PHASE_AA_SWAPPED = 3 };
 
+// The share of a two-step launch's lanes and planes that must be the domain's
+// own for it to be taken.  Single steps / pairs, us per step, BGK (MRT):
+//   FP64  96^3 (0.52) 46 / 48 (46 / 52)   112^3 (0.66) 84 / 70 (83 / 75)
+//        130^3 (0.54) 130 / 127 (129 / 138)   256^3 (0.90) 983 / 630 (988 / 680)
+//   FP32  80^3 (0.34) 18 / 18 (17 / 19)   96^3 28 / 21   130^3 65 / 63   256^3 484 / 290
+constexpr double PAIR_FILL_F64 = 0.6, PAIR_FILL_F32 = 0.5;
+
 size_t elem_size(int storage) { return storage == HLBM_F64 ? 8 : (storage == HLBM_F32 ? 4 : 2); }
 
 }  // namespace
@@ -80,6 +87,7 @@ struct hlbm_domain {
   int xcd_remap = 1;
   int npt = 1;
   int force_wide = 0;
+  int pairs = 1;    // two steps per pass where it applies: 0 never, 1 large domains, 2 any size
   int variant = 0;  // bulk-kernel variant (hlbm_set_launch)
   int boundary_first = 1;  // program-plane kernel before the bulk kernel (measured 1-2 % faster)
   // the program-plane kernel on a second stream beside the bulk kernel
@@ -391,6 +399,30 @@ static int launch(hlbm_domain* h, int mode, bool write_macro, hipStream_t s, voi
   return HLBM_OK;
 }
 
+// Two steps in one pass (pair_kernel): domains whose every node runs the plain
+// pull, collide, store, and large enough to fill the chip with its tiles.
+static bool steps_in_pairs(const hlbm_domain* h, const StepParams& p, PairGrid* g) {
+  if (!h->pairs || h->d.pattern != HLBM_PATTERN_AB) return false;
+  if (h->d.storage != HLBM_F64 && h->d.storage != HLBM_F32) return false;
+  if (h->any_wall || p.nprog || p.prog_planes || p.nset || p.nspec || !default_layout_p(h)) return false;
+  if (!p.pair32 || wide_offsets(p, h->esize)) return false;
+  const double fill = h->d.storage == HLBM_F64 ? PAIR_FILL_F64 : PAIR_FILL_F32;
+  int64_t cost;
+  *g = pair_grid(h->nx, h->ny, h->nz, &cost);
+  return h->pairs == 2 || (double)h->N >= fill * (double)cost * (PAIR_TX * PAIR_TY);
+}
+
+static int launch_pair(hlbm_domain* h, StepParams& p, const PairGrid& g, bool write_macro, hipStream_t s) {
+  p.fin = h->buf[h->cur];
+  p.fout = h->buf[h->cur ^ 1];
+  p.write_macro = write_macro ? 1 : 0;
+  const int coll = h->d.collision == HLBM_MRT ? COLL_MRT : COLL_BGK;
+  const hipError_t e = h->d.storage == HLBM_F64 ? launch_pair_f64(coll, g, p, s) : launch_pair_f32(coll, g, p, s);
+  if (e != hipSuccess) return fail(HLBM_ERR_HIP, std::string("step pair launch: ") + hipGetErrorString(e));
+  h->cur ^= 1;
+  return HLBM_OK;
+}
+
 // Bring the state to the reference's post-stream/post-BC form f^T.
 static int materialize(hlbm_domain* h, hipStream_t s) {
   if (h->phase == PHASE_POST) {
@@ -474,6 +506,7 @@ int hlbm_domain_create(const hlbm_domain_desc* desc, hlbm_domain** out) {
   if (const char* np = getenv("HLBM_NPT")) h->npt = atoi(np) == 2 ? 2 : 1;
   // the 64-bit-address variant otherwise runs only on domains above 2^32 bytes per plane
   if (const char* fw = getenv("HLBM_FORCE_WIDE")) h->force_wide = atoi(fw) ? 1 : 0;
+  if (const char* pr = getenv("HLBM_PAIRS")) h->pairs = std::max(0, std::min(2, atoi(pr)));
   if (const char* bf = getenv("HLBM_BOUNDARY_FIRST")) h->boundary_first = atoi(bf) ? 1 : 0;
   if (const char* ov = getenv("HLBM_OVERLAP")) h->overlap = atoi(ov) ? 1 : 0;
   (void)hipGetDevice(&h->device);
@@ -1051,6 +1084,17 @@ int hlbm_step(hlbm_domain* h, int32_t nsteps, uint32_t flags, void* stream) {
       if (rc) return rc;
       h->phase = even ? PHASE_AA_SWAPPED : PHASE_AA_PENDING;
     } else {
+      if (h->phase == PHASE_POST && k + 2 <= nsteps) {
+        StepParams p = base_params(h);
+        PairGrid g;
+        if (steps_in_pairs(h, p, &g)) {
+          const int rc = launch_pair(h, p, g, (flags & HLBM_STEP_WRITE_MACRO) && k + 2 == nsteps, s);
+          if (rc) return rc;
+          h->t += 2;
+          k++;
+          continue;
+        }
+      }
       const int mode = h->phase == PHASE_PRE ? MODE_COLLIDE : MODE_FUSED;
       int rc = launch(h, mode, wm, s);
       if (rc) return rc;

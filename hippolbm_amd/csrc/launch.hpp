@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include "fp32_constants.hpp"
+#include "pair_kernel.hpp"
 #include "step_kernel.hpp"
 
 namespace hlbm {
@@ -124,6 +125,18 @@ hipError_t step_dispatch(int coll, int mode, int npt, dim3 grid, dim3 block, con
   if (mode == MODE_FUSED) return step_go_npt<S, COLL_MRT, MODE_FUSED>(npt, grid, block, p, s);
   return step_go_npt<S, COLL_MRT, MODE_COLLIDE>(npt, grid, block, p, s);
 }
+
+template <class S>
+hipError_t pair_go(int coll, const PairGrid& g, const StepParams& p, hipStream_t s) {
+  const dim3 grid((unsigned)(g.tx * g.ty * g.segs)), block((PAIR_TY + 3) * 64);
+  if (coll == COLL_BGK)
+    hipLaunchKernelGGL((pair_kernel<S, COLL_BGK>), grid, block, 0, s, p, g);
+  else
+    hipLaunchKernelGGL((pair_kernel<S, COLL_MRT>), grid, block, 0, s, p, g);
+  return hipGetLastError();
+}
+hipError_t launch_pair_f64(int coll, const PairGrid& g, const StepParams& p, hipStream_t s);
+hipError_t launch_pair_f32(int coll, const PairGrid& g, const StepParams& p, hipStream_t s);
 
 // FP64 storage, FP64 compute, no contraction (step_f64.hip)
 hipError_t launch_step_f64(int coll, int mode, int npt, dim3 grid, dim3 block, const StepParams& p, hipStream_t s);

@@ -1,0 +1,292 @@
+// pair_kernel.hpp -- two time steps in one pass over the populations (gfx950).
+//
+// A step of a large domain is bound by the traffic of 19 population planes in
+// and 19 out: on MI355X that pattern alone, without any arithmetic, runs at
+// 5.1-5.5 TB/s, which is what step_kernel reaches, while its FP64 BGK
+// arithmetic takes a fifth of that time.  So this kernel does two steps per
+// read and write of the lattice.
+//
+// A workgroup owns TX x TY columns and walks a segment of planes upwards.  Per
+// plane s every thread gathers its node from HBM and collides it (step one), on
+// the tile and on a ring of one node around it; the post-collision populations
+// then meet in LDS, and the tile's threads pull, collide and store plane s - 1
+// (step two).  Populations are pulled one plane up, level or one plane down:
+//   c_z = -1 of plane s       written before the first barrier,
+//   c_z =  0 of plane s - 1   written in the iteration before,
+//   c_z = +1 of plane s - 2   kept in registers for an iteration, then written,
+// so each of the 16 directions that leave the column needs one buffer only, and
+// the three that stay in it (rest, +z, -z) need none.  FP32 has room for more:
+// two sets of buffers, used in turn, which leaves one barrier per plane, and
+// registers for the next plane's loads, issued before step two.  (In FP64 those
+// loads spill: 512^3 4.7 ms per step without them, 8.9 ms with.)
+//
+// A node whose upstream neighbour is outside a non-periodic face pushes its own
+// opposite population (plus the moving-wall term) into the slot it will pull
+// from; that slot belongs to a node outside the domain, which nobody else
+// writes.  The arithmetic per node and step is the single step's own code, so
+// populations are the same bit for bit.
+//
+// Taken by domains without walls, boundary programs and start_iteration boxes,
+// in FP64 and FP32 storage (16-bit storage rounds between the steps and is near
+// its issue limit).
+#pragma once
+
+#include "step_kernel.hpp"
+
+namespace hlbm {
+
+constexpr int PAIR_TX = 64;  // tile columns along x: one wave per row
+// Tile rows: with the ring's two rows and the wave for its columns, the 16 waves
+// a workgroup can have.  The ring is stepped twice, so a step costs 16/13 of its
+// arithmetic (9 rows: 512^3 FP64 5.1-5.4 ms per step instead of 4.7).
+constexpr int PAIR_TY = 13;
+
+struct PairGrid {
+  int32_t tx, ty, segs;  // tiles along x and y, segments along z
+  int32_t planes;        // planes per segment
+};
+
+// The segments that cost the fewest planes: a CU holds one workgroup at a time
+// (registers and LDS), and each segment steps a plane more on either side.
+// `cost` is that number of planes times `cus`: the planes the chip steps,
+// against nx * ny * nz / (64 * 13) for a grid that fills it exactly.
+constexpr int PAIR_CUS = 256;
+inline PairGrid pair_grid(int nx, int ny, int nz, int64_t* cost) {
+  PairGrid g{(nx + PAIR_TX - 1) / PAIR_TX, (ny + PAIR_TY - 1) / PAIR_TY, 1, nz};
+  *cost = INT64_MAX;
+  for (int k = 1; k <= nz; k++) {
+    const int planes = (nz + k - 1) / k, segs = (nz + planes - 1) / planes;
+    const int64_t rounds = ((int64_t)g.tx * g.ty * segs + PAIR_CUS - 1) / PAIR_CUS;
+    const int64_t c = rounds * (planes + 2) * PAIR_CUS;
+    if (c < *cost) {
+      *cost = c;
+      g.planes = planes;
+      g.segs = segs;
+    }
+  }
+  return g;
+}
+
+// LDS slot of a direction that leaves its column, in the order c_z = 0, +1, -1.
+HLBM_HD constexpr int pair_slot(int i) {
+  constexpr int s[Q] = {-1, 0, 1, 2, 3, -1, -1, 4, 5, 6, 7, 8, 12, 13, 9, 10, 14, 15, 11};
+  return s[i];
+}
+
+// Barrier for the LDS buffers alone: loads and stores of populations stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <class S, int COLL>
+__global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepParams p, const PairGrid g) {
+  using O = StoreOps<S>;
+  using C = typename O::C;
+  constexpr int TY = PAIR_TY, R = TY + 2, W = PAIR_TX + 2;
+  constexpr bool AHEAD = sizeof(S) == 4;    // the next plane's loads before step two
+  constexpr int BUFS = sizeof(S) == 4 ? 2 : 1;
+  __shared__ C buf[BUFS][16][R][W];
+
+  // tiles next to each other in y run on the same XCD at the same time: they
+  // share the rows between them
+  const uint32_t nt = (uint32_t)(g.tx * g.ty * g.segs);
+  uint32_t t = blockIdx.x;
+  {
+    const uint32_t per = nt / 8u;
+    if (t < per * 8u) t = (t % 8u) * per + t / 8u;
+  }
+  const int ty = (int)(t % (uint32_t)g.ty);
+  const uint32_t t2 = t / (uint32_t)g.ty;
+  const int tx = (int)(t2 % (uint32_t)g.tx), seg = (int)(t2 / (uint32_t)g.tx);
+
+  const int nx = p.nx, ny = p.ny, nz = p.nz;
+  const bool px = p.per[0] != 0, py = p.per[1] != 0, pz = p.per[2] != 0;
+  const int wx = min(PAIR_TX, nx - tx * PAIR_TX), hy = min(TY, ny - ty * TY);  // this tile's columns and rows
+  const int zs = seg * g.planes, ze = min(zs + g.planes, nz);
+
+  // rows 0 .. TY + 1 are a wave each (0 and hy + 1 the ring's); the last wave
+  // holds the ring's columns left and right of every row
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63u);
+  const bool side = wave == R;
+  const int r = side ? lane >> 1 : wave;
+  const int c = side ? ((lane & 1) ? wx + 1 : 0) : lane + 1;
+  int x = tx * PAIR_TX + c - 1, y = ty * TY + r - 1;
+  bool act = r <= hy + 1 && c <= wx + 1 && (side || c <= wx);
+  if (x < 0 || x >= nx) {
+    act = act && px;
+    x = x < 0 ? nx - 1 : 0;
+  }
+  if (y < 0 || y >= ny) {
+    act = act && py;
+    y = y < 0 ? ny - 1 : 0;
+  }
+  const bool mine = !side && r >= 1 && r <= hy && c <= wx;  // the tile's own columns
+
+  // the node's neighbours outside a non-periodic face
+  const bool fxm = !px && x == 0, fxp = !px && x == nx - 1, fym = !py && y == 0, fyp = !py && y == ny - 1;
+  const bool wave_face = __any(act && (fxm || fxp || fym || fyp));
+
+  // byte offsets inside a plane: of the rows and columns populations come from,
+  // added where they are used (nine sums kept across the loop would spill)
+  const uint32_t nxy = (uint32_t)nx * (uint32_t)ny;
+  const uint32_t unit = (uint32_t)sizeof(S), row = (uint32_t)nx * unit;
+  const uint32_t xo[3] = {(uint32_t)(x > 0 ? x - 1 : (px ? nx - 1 : 0)) * unit, (uint32_t)x * unit,
+                          (uint32_t)(x < nx - 1 ? x + 1 : (px ? 0 : x)) * unit};
+  const uint32_t yo[3] = {(uint32_t)(y > 0 ? y - 1 : (py ? ny - 1 : 0)) * row, (uint32_t)y * row,
+                          (uint32_t)(y < ny - 1 ? y + 1 : (py ? 0 : y)) * row};
+  auto off = [&](int b, int a) { return yo[b] + lane_offset(xo[a]); };
+
+  const S* __restrict__ fin = (const S*)p.fin;
+  auto plane_valid = [&](int s) { return pz || (s >= 0 && s < nz); };
+  auto wrapped = [&](int s) { return s < 0 ? s + nz : (s >= nz ? s - nz : s); };
+
+  // direction i's upstream node is outside a non-periodic face (zout: a z face)
+  auto outside = [&](auto ic, bool zout) {
+    constexpr int i = decltype(ic)::value;
+    bool o = zout;
+    if constexpr (CX(i) != 0) o = o || (CX(i) == 1 ? fxm : fxp);
+    if constexpr (CY(i) != 0) o = o || (CY(i) == 1 ? fym : fyp);
+    return o;
+  };
+  // step one's populations arriving at the node in plane s
+  auto gather = [&](int s, C* f) {
+    const int z = wrapped(s);
+    if (!pz && (z == 0 || z == nz - 1)) {
+      const NodeNbrs a = node_nbrs<S>(p, x, y, z);
+      gather_select<S, MODE_FUSED>(p, (uint32_t)z * nxy * (uint32_t)sizeof(S) + off(1, 1), a, 0u, f);
+    } else if (wave_face) {
+      // as gather_select: a lane whose upstream node is outside takes its own
+      // opposite population, both addressed from the first plane of the pair
+      const uint32_t stb = (uint32_t)(p.stride * sizeof(S)), pb = nxy * (uint32_t)sizeof(S);
+      const uint32_t zo[3] = {(uint32_t)wrapped(z - 1) * pb, (uint32_t)z * pb, (uint32_t)wrapped(z + 1) * pb};
+      f[0] = O::ld(at_bytes(scalar_ptr(fin), lane_offset(off(1, 1) + zo[1])), 0);
+      const S* b = fin;
+      static_for<1, Q>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        constexpr int lo = (i & 1) ? i : i - 1;
+        if constexpr (i & 1) b = scalar_ptr(b + (size_t)(i == 1 ? 1 : 2) * p.stride);
+        uint32_t o = off(1 - CY(i), 1 - CX(i)) + ((uint32_t)(i - lo) * stb + zo[1 - CZ(i)]);
+        if constexpr (CX(i) != 0 || CY(i) != 0) {
+          const uint32_t own = off(1, 1) + ((uint32_t)(OPP(i) - lo) * stb + zo[1]);
+          o = outside(ic, false) ? own : o;
+        }
+        f[i] = O::ld(at_bytes(b, o), 0);
+      });
+    } else {
+      const size_t zo[3] = {(size_t)wrapped(z - 1) * nxy, (size_t)z * nxy, (size_t)wrapped(z + 1) * nxy};
+      const S* b = fin;
+      static_for([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        b = scalar_ptr(i ? b + p.stride : b);
+        const S* q = scalar_ptr(b + zo[1 - CZ(i)]);
+        f[i] = O::ld(at_bytes(q, lane_offset(off(1 - CY(i), 1 - CX(i)))), 0);
+      });
+    }
+  };
+  auto wall_term = [&](auto ic, bool zout) -> C {
+    constexpr int i = decltype(ic)::value;
+    if constexpr (CZ(i) == 0) {
+      return C(0);
+    } else {
+      constexpr int sd = CZ(i) == 1 ? 0 : 1;
+      return zout && p.cav_gather && p.cav_on[sd] ? cav_coef<C>(p, sd, cavity_slot(i)) : C(0);
+    }
+  };
+
+  C gn[Q];              // arriving in plane s
+  C up[4] = {}, h0 = C(0), h5 = C(0), u5 = C(0);  // kept: c_z = +1 and rest of plane s - 1, +z of plane s - 2
+  if (AHEAD && act && plane_valid(zs - 1)) gather(zs - 1, gn);
+  for (int s = zs - 1; s <= ze; s++) {
+    const bool valid = plane_valid(s), before = plane_valid(s - 1);
+    auto& lds = buf[BUFS == 2 ? s & 1 : 0];
+    auto& next = buf[BUFS == 2 ? ~s & 1 : 0];  // read by the next iteration
+    C f[Q];
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int i = 0; i < Q; i++) f[i] = gn[i];
+    } else {
+      if (act && valid) gather(s, f);
+    }
+    if (act && valid) {
+      collide_node<S, COLL, MODE_FUSED, false, false>(p, 0u, false, f);
+      // these reach step two in registers, rounded as the others are by LDS
+      f[0] = rounded(f[0]);
+      f[5] = rounded(f[5]);
+      f[6] = rounded(f[6]);
+    }
+    if (AHEAD && s < ze && act && plane_valid(s + 1)) gather(s + 1, gn);
+
+    // c_z = -1 of plane s; on a face, of plane s - 1's own bounce-back
+    if (act && valid) {
+      static_for<1, Q>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        if constexpr (CZ(i) == -1 && pair_slot(i) >= 0) lds[pair_slot(i)][r][c] = f[i];
+      });
+    }
+    const bool top = !pz && s == nz;  // plane s - 1 lies on the high z face
+    if (mine && before && (wave_face || top)) {
+      static_for<1, Q>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        if constexpr (CZ(i) == -1 && pair_slot(i) >= 0) {
+          if (outside(ic, top)) lds[pair_slot(i)][r - CY(i)][c - CX(i)] = up[pair_slot(OPP(i)) - 8] + wall_term(ic, top);
+        }
+      });
+    }
+    lds_barrier();
+
+    // step two: plane s - 1
+    if (s > zs && mine) {
+      const int z = s - 1;
+      C f2[Q];
+      f2[0] = h0;
+      f2[5] = u5;
+      f2[6] = top ? h5 + wall_term(std::integral_constant<int, 6>{}, true) : f[6];
+      static_for<1, Q>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        if constexpr (pair_slot(i) >= 0) f2[i] = lds[pair_slot(i)][r - CY(i)][c - CX(i)];
+      });
+      const uint32_t idx = (uint32_t)z * nxy + off(1, 1) / (uint32_t)sizeof(S);
+      collide_node<S, COLL, MODE_FUSED>(p, idx, false, f2);
+      S* b = (S*)p.fout + (size_t)z * nxy;
+      const uint32_t bo = lane_offset(off(1, 1));
+      static_for([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        b = scalar_ptr(i ? b + p.stride : b);
+        O::st(at_bytes(b, bo), 0, f2[i]);
+      });
+    }
+    if constexpr (BUFS == 1) lds_barrier();
+
+    // c_z = 0 of plane s, c_z = +1 of plane s - 1; on a face, of plane s's own bounce-back
+    const bool bottom = !pz && s == 0;
+    if (act) {
+      static_for<1, Q>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        if constexpr (pair_slot(i) >= 0) {
+          if (CZ(i) == 0 && valid) next[pair_slot(i)][r][c] = f[i];
+          if (CZ(i) == 1 && before) next[pair_slot(i)][r][c] = up[pair_slot(i) - 8];
+        }
+      });
+    }
+    if (mine && valid && (wave_face || bottom)) {
+      static_for<1, Q>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        if constexpr (pair_slot(i) >= 0 && CZ(i) >= 0) {
+          const bool zout = CZ(i) == 1 && bottom;
+          if (outside(ic, zout)) next[pair_slot(i)][r - CY(i)][c - CX(i)] = f[OPP(i)] + wall_term(ic, zout);
+        }
+      });
+    }
+    u5 = bottom ? f[6] + wall_term(std::integral_constant<int, 5>{}, true) : h5;
+    h5 = f[5];
+    h0 = f[0];
+    static_for<1, Q>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      if constexpr (CZ(i) == 1 && pair_slot(i) >= 0) up[pair_slot(i) - 8] = f[i];
+    });
+  }
+}
+
+}  // namespace hlbm

@@ -9,6 +9,10 @@ hipError_t launch_step_f64(int coll, int mode, int npt, dim3 grid, dim3 block, c
   return step_dispatch<double>(coll, mode, npt, grid, block, p, s);
 }
 
+hipError_t launch_pair_f64(int coll, const PairGrid& g, const StepParams& p, hipStream_t s) {
+  return pair_go<double>(coll, g, p, s);
+}
+
 hipError_t launch_batch_f64(int coll, unsigned blocks, const BatchParams& bp, hipStream_t s) {
   if (coll == COLL_BGK)
     hipLaunchKernelGGL((batch_kernel<double, COLL_BGK>), dim3(blocks), dim3(256), 0, s, bp);

@@ -408,6 +408,14 @@ __device__ __forceinline__ void moments_f32(const float* g, float& dr, float& jx
   });
 }
 
+// A value the optimizer cannot look behind: no multiplication before it is
+// contracted with an addition after it.
+template <class C>
+__device__ __forceinline__ C rounded(C v) {
+  asm("" : "+v"(v));
+  return v;
+}
+
 // 1 / x for x near 1 (a lattice density): the hardware reciprocal (1 ulp)
 // and one Newton step, which leaves it within half an ulp plus a few units of
 // 2^-46; three instructions instead of the IEEE division's eleven.
@@ -913,8 +921,8 @@ __device__ __forceinline__ void apply_program(const StepParams& p, int x, int y,
 // Phase 3: macro_variables (optionally written out) and collision.
 // RAW (FP16 BGK in the A/B bulk paths only): the populations leave already
 // multiplied by the storage scale, for store_bulk<..., RAW>; wall lanes are
-// scaled as they are.
-template <class S, int COLL, int MODE, bool RAW = false>
+// scaled as they are.  MACRO: rho and u are written out when the step asks for it.
+template <class S, int COLL, int MODE, bool RAW = false, bool MACRO = true>
 __device__ __forceinline__ void collide_node(const StepParams& p, uint32_t idx, bool wall,
                                              typename StoreOps<S>::C* f) {
   using O = StoreOps<S>;
@@ -923,7 +931,7 @@ __device__ __forceinline__ void collide_node(const StepParams& p, uint32_t idx, 
     if constexpr (!SHIFT) {
       double rho, ux, uy, uz;
       macro_f64((const double*)f, rho, ux, uy, uz);
-      if (p.write_macro) {
+      if (MACRO && p.write_macro) {
         if (!wall) {
           p.m0[idx] = rho;
           p.m1[idx] = ux;
@@ -952,8 +960,10 @@ __device__ __forceinline__ void collide_node(const StepParams& p, uint32_t idx, 
       moments_f32((const float*)f, dr, jx, jy, jz);
       const float rho = 1.0f + dr;
       const float inv = recip_f32(rho);
-      const float ux = jx * inv, uy = jy * inv, uz = jz * inv;
-      if (p.write_macro) {
+      // rounded here in every kernel: without the barriers a sum u_x + u_y in the
+      // same basic block could take an unrounded product (contraction)
+      const float ux = rounded(jx * inv), uy = rounded(jy * inv), uz = rounded(jz * inv);
+      if (MACRO && p.write_macro) {
         if (!wall) {
           p.m0[idx] = (double)rho;
           p.m1[idx] = (double)ux;

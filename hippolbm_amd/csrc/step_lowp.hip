@@ -18,6 +18,10 @@ hipError_t launch_step_lowp(int storage, int coll, int mode, int npt, dim3 grid,
   }
 }
 
+hipError_t launch_pair_f32(int coll, const PairGrid& g, const StepParams& p, hipStream_t s) {
+  return pair_go<float>(coll, g, p, s);
+}
+
 template <class S>
 static hipError_t batch_one(int coll, unsigned blocks, const BatchParams& bp, hipStream_t s) {
   if (coll == COLL_BGK)
