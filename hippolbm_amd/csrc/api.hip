@@ -96,6 +96,7 @@ struct hlbm_domain {
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   int device = 0;
   uint64_t bytes = 0;
+  TransferRing* ring = nullptr;  // pinned slots of large transfers to and from host arrays
   NodeLayout lay{};  // node layout in HBM (hlbm_set_layout; default x fastest)
 };
 
@@ -568,6 +569,7 @@ int hlbm_domain_destroy(hlbm_domain* h) {
   if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
   if (h->ev_join) (void)hipEventDestroy(h->ev_join);
   if (h->side) (void)hipStreamDestroy(h->side);
+  free_ring(h->ring);
   delete h;
   return HLBM_OK;
 }
@@ -937,7 +939,7 @@ int hlbm_set_populations_f64(hlbm_domain* h, const double* f, int32_t layout) {
   {
     const auto planes = population_planes(h, f, layout);
     hipError_t e = hipSuccess;
-    const int t = planes_to_device(transfer_grid(h, layout), planes.data(), Q, 0, &e);
+    const int t = planes_to_device(&h->ring, transfer_grid(h, layout), planes.data(), Q, 0, &e);
     if (t == TRANSFER_FAILED) return fail(HLBM_ERR_HIP, std::string("populations in: ") + hipGetErrorString(e));
     if (t == TRANSFER_DONE) {
       HIP_TRY(hipDeviceSynchronize());
@@ -1030,7 +1032,7 @@ int hlbm_get_populations_f64(hlbm_domain* h, double* f, int32_t layout) {
   {
     const auto planes = population_planes(h, f, layout);
     hipError_t e = hipSuccess;
-    const int t = planes_to_host(transfer_grid(h, layout), planes.data(), Q, 0, &e);
+    const int t = planes_to_host(&h->ring, transfer_grid(h, layout), planes.data(), Q, 0, &e);
     if (t == TRANSFER_FAILED) return fail(HLBM_ERR_HIP, std::string("populations out: ") + hipGetErrorString(e));
     if (t == TRANSFER_DONE) {
       if (layout == HLBM_LAYOUT_REF) fill_periodic_ghosts(h, f, Q);
@@ -1126,7 +1128,7 @@ static int copy_macro_out(hlbm_domain* h, double* rho, double* u, int32_t layout
     for (int c = 0; u && c < 3; c++)
       p[n++] = NodePlane{h->m1 + c * N, u + c * (layout == HLBM_LAYOUT_REF ? ref_count(h) : N), -1};
     hipError_t e = hipSuccess;
-    const int t = planes_to_host(transfer_grid(h, layout), p, n, 0, &e);
+    const int t = planes_to_host(&h->ring, transfer_grid(h, layout), p, n, 0, &e);
     if (t == TRANSFER_FAILED) return fail(HLBM_ERR_HIP, std::string("rho and u out: ") + hipGetErrorString(e));
     if (t == TRANSFER_DONE) return HLBM_OK;
   }

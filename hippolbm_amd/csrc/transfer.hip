@@ -10,13 +10,15 @@
 // order at the link's rate (53 GB/s to the host, 55 from it; conversion and
 // layout cost nothing there), and a few threads move it between the slots and
 // the caller's array, both sides running ahead of each other by half a ring.
+// The ring stays with the domain: the first touch of pinned memory costs 0.4 ms
+// a MiB, and a ring made anew by each call paid it in every other one.  Slots of
+// 512 KiB leave the link at 47 GB/s, 1 MiB (for 64 MiB and more) at 50.
 // Measured against copies plane by plane through the runtime: 400 steps of the
 // porous channel 256 x 128 x 128 (layout "yzx") with rho and u read 215 -> 105
 // ms, 300 MRT steps of 128^3 FP32 35.5 -> 20.2 ms, populations of 96^3 in and
 // out 18.5 -> 9.3 ms.
 //
-// The slots and threads live as long as the call (a pinned allocation of this
-// size costs about 20 us once the process has had one).
+// Threads live as long as the call.
 #include <algorithm>
 #include <condition_variable>
 #include <cstring>
@@ -31,12 +33,44 @@
 #include "transfer.hpp"
 
 namespace hlbm {
+
+constexpr size_t SLOT_SMALL = (size_t)512 << 10, SLOT_LARGE = (size_t)1 << 20, LARGE_FROM = (size_t)64 << 20;
+constexpr int SLOTS = 16, THREADS = 8;
+
+struct TransferRing {
+  double* mem = nullptr;
+  size_t slot_bytes = 0;
+  hipEvent_t ev[SLOTS] = {};
+  explicit TransferRing(size_t bytes) : slot_bytes(bytes) {}
+  ~TransferRing() {
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (mem) (void)hipHostFree(mem);
+  }
+  bool open() {
+    if (hipHostMalloc((void**)&mem, slot_bytes * SLOTS, hipHostMallocCoherent) != hipSuccess) {
+      mem = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+    for (int k = 0; k < SLOTS; k++)
+      if (hipEventCreateWithFlags(&ev[k], hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
+        ev[k] = nullptr;
+        return false;
+      }
+    return true;
+  }
+};
+
+void free_ring(TransferRing* ring) { delete ring; }
+
 namespace {
 
-// Smaller transfers gain nothing over the runtime's own copies.
-constexpr size_t TRANSFER_MIN_BYTES = (size_t)4 << 20;
-constexpr size_t SLOT_MAX = (size_t)1 << 20, SLOT_MIN = (size_t)256 << 10;
-constexpr int SLOTS = 16, THREADS = 8;
+// Below these sizes the runtime's own copies of whole planes are as fast (to the
+// host 10 MiB 0.67 ms and 0.70 through the ring, 25 MiB 2.0 and 1.4; from warm
+// host pages 25 MiB 1.3 either way, 38 MiB 1.9 and 1.6), unless every plane has
+// to be rearranged on the host.
+constexpr size_t MIN_TO_HOST = (size_t)12 << 20, MIN_TO_DEVICE = (size_t)32 << 20, MIN_REARRANGED = (size_t)4 << 20;
 
 // node k of the host's order (x fastest) -> index in the device layout
 struct NodeOrder {
@@ -189,42 +223,31 @@ class Copiers {
   std::vector<std::thread> pool_;
 };
 
-// The pinned ring and its events, given back on every way out.
-struct Ring {
-  double* mem = nullptr;
-  hipEvent_t ev[SLOTS] = {};
-  ~Ring() {
-    for (hipEvent_t e : ev)
-      if (e) (void)hipEventDestroy(e);
-    if (mem) (void)hipHostFree(mem);
-  }
-  bool open(size_t bytes, int slots) {
-    if (hipHostMalloc((void**)&mem, bytes * slots, hipHostMallocCoherent) != hipSuccess) {
-      mem = nullptr;
-      (void)hipGetLastError();
-      return false;
-    }
-    for (int k = 0; k < slots; k++)
-      if (hipEventCreateWithFlags(&ev[k], hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
-        ev[k] = nullptr;
-        return false;
-      }
-    return true;
-  }
-};
-
-int transfer(bool out, const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s, hipError_t* err) {
+int transfer(TransferRing** owned, bool out, const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s, hipError_t* err) {
   *err = hipSuccess;
   const uint32_t N = (uint32_t)g.n[0] * (uint32_t)g.n[1] * (uint32_t)g.n[2];
   const size_t total = (size_t)N * 8 * count;
-  if (total < TRANSFER_MIN_BYTES) return TRANSFER_DECLINED;
-  const size_t slot_bytes = std::min(SLOT_MAX, std::max(SLOT_MIN, total / 32 / 4096 * 4096));
-  const uint32_t per = (uint32_t)(slot_bytes / 8);
+  const bool perm = !(g.lay.ord[0] == 0 && g.lay.ord[1] == 1);
+  if (total < (perm || g.reference ? MIN_REARRANGED : out ? MIN_TO_HOST : MIN_TO_DEVICE)) return TRANSFER_DECLINED;
+  if (*owned && total >= LARGE_FROM && (*owned)->slot_bytes < SLOT_LARGE) {
+    delete *owned;
+    *owned = nullptr;
+  }
+  if (!*owned) {
+    *owned = new TransferRing(total >= LARGE_FROM ? SLOT_LARGE : SLOT_SMALL);
+    if (!(*owned)->open()) {
+      delete *owned;
+      *owned = nullptr;
+      return TRANSFER_DECLINED;
+    }
+  }
+  TransferRing& ring = **owned;
+  const uint32_t per = (uint32_t)(ring.slot_bytes / 8);
+  constexpr int slots = SLOTS, ahead = SLOTS / 2;
   std::vector<Chunk> chunks;
   for (int p = 0; p < count; p++)
     for (uint32_t a = 0; a < N; a += per) chunks.push_back({p, a, std::min(per, N - a)});
-  const int nc = (int)chunks.size(), slots = std::min(SLOTS, nc), ahead = slots / 2;
-  if (ahead < 1) return TRANSFER_DECLINED;
+  const int nc = (int)chunks.size();
 
   NodeOrder o;
   o.nx = (uint32_t)g.n[0];
@@ -232,16 +255,14 @@ int transfer(bool out, const TransferGrid& g, const NodePlane* planes, int count
   node_divisor(o.nx, o.div.m0, o.div.s0);
   node_divisor(o.nxy, o.div.m01, o.div.s01);
   o.lay = g.lay;
-  const bool perm = !(g.lay.ord[0] == 0 && g.lay.ord[1] == 1);
 
-  Ring ring;
-  if (!ring.open(slot_bytes, slots)) return TRANSFER_DECLINED;
   auto slot = [&](int c) { return ring.mem + (size_t)(c % slots) * per; };
   Copiers copiers(nc, [&](int c) {
     const Chunk& k = chunks[c];
     copy_rows(g, out, slot(c), planes[k.plane].host, k.first, k.n);
   });
-  if (!copiers.start(std::min(THREADS, nc))) return TRANSFER_DECLINED;
+  // about 2 MiB of copying pays for a thread
+  if (!copiers.start((int)std::min<size_t>(THREADS, total >> 21))) return TRANSFER_DECLINED;
 
   auto device = [&](int c) -> hipError_t {
     const Chunk& k = chunks[c];
@@ -288,15 +309,15 @@ int transfer(bool out, const TransferGrid& g, const NodePlane* planes, int count
       }
     }
   }
-  // nothing may still read or write the slots when they are freed
+  // nothing may still read or write the slots afterwards
   const hipError_t last = hipStreamSynchronize(s);
   *err = e != hipSuccess ? e : last;
   return *err == hipSuccess ? TRANSFER_DONE : TRANSFER_FAILED;
 }
 
-int guarded(bool out, const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s, hipError_t* err) {
+int guarded(TransferRing** ring, bool out, const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s, hipError_t* err) {
   try {
-    return transfer(out, g, planes, count, s, err);
+    return transfer(ring, out, g, planes, count, s, err);
   } catch (const std::bad_alloc&) {  // before any work: the lists and threads come first
     *err = hipErrorOutOfMemory;
     return TRANSFER_FAILED;
@@ -305,11 +326,13 @@ int guarded(bool out, const TransferGrid& g, const NodePlane* planes, int count,
 
 }  // namespace
 
-int planes_to_host(const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s, hipError_t* err) {
-  return guarded(true, g, planes, count, s, err);
+int planes_to_host(TransferRing** ring, const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s,
+                   hipError_t* err) {
+  return guarded(ring, true, g, planes, count, s, err);
 }
-int planes_to_device(const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s, hipError_t* err) {
-  return guarded(false, g, planes, count, s, err);
+int planes_to_device(TransferRing** ring, const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s,
+                     hipError_t* err) {
+  return guarded(ring, false, g, planes, count, s, err);
 }
 
 }  // namespace hlbm

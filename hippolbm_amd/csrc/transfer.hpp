@@ -30,13 +30,20 @@ struct TransferGrid {
   RestShift shift;
 };
 
+// The pinned slots of a domain's transfers: made by its first large one, kept
+// until the domain is destroyed (8 MiB, 16 MiB for 64 MiB and more).
+struct TransferRing;
+void free_ring(TransferRing* ring);
+
 enum TransferStatus { TRANSFER_DONE = 0, TRANSFER_DECLINED = 1, TRANSFER_FAILED = 2 };
 
 // Copies all planes, in order, and returns when the host (device) arrays are
 // complete.  Kernels run on `s`; *err holds the HIP error when FAILED.
 // DECLINED: nothing was done (the arrays are too small for it to pay, or no
 // pinned memory or thread could be had); the caller copies plane by plane.
-int planes_to_host(const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s, hipError_t* err);
-int planes_to_device(const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s, hipError_t* err);
+int planes_to_host(TransferRing** ring, const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s,
+                   hipError_t* err);
+int planes_to_device(TransferRing** ring, const TransferGrid& g, const NodePlane* planes, int count, hipStream_t s,
+                     hipError_t* err);
 
 }  // namespace hlbm

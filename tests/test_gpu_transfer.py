@@ -1,8 +1,9 @@
 """Populations, density and velocity between the device and host arrays, at
-sizes around the one from which they go through the pinned ring (4 MiB in all:
-131072 nodes for rho and u, 27595 for populations): one ring's worth of chunks,
-rows and planes that straddle chunks, more chunks than slots, a device layout
-other than the host's, the reference layout with its ghost layers, each storage.
+sizes around the ones from which they go through the pinned ring (rearranged
+planes 4 MiB in all, others 12 MiB to the host and 32 MiB to the device): a ring
+not filled once, rows and planes that straddle chunks, more chunks than slots,
+the larger slots from 64 MiB on, a device layout other than the host's, the
+reference layout with its ghost layers, each storage.
 
 Exact: the host form of a stored population is a fixed sequence of IEEE
 operations, restated here in numpy."""
@@ -29,9 +30,10 @@ def stored(f, storage):
     return g.astype(np.float64) + w
 
 
-# 30 x 30 x 30 and 31 x 30 x 30: either side of the populations' size;
-# 64 x 64 x 32 and 64 x 64 x 31: either side of the fields'; odd rows; more than one round of the ring
-SIZES = [(30, 30, 30), (31, 30, 30), (64, 64, 31), (64, 64, 32), (131, 67, 61), (129, 130, 131)]
+# 30 x 30 x 30 and 31 x 30 x 30, 43^3 and 44^3: either side of the populations' 4 and 12 MiB; 64 x 64 x 31 and
+# 64 x 64 x 32: of the fields' 4 MiB; 59^3 and 61^3: of 32 MiB to the device; odd rows; 64 MiB and more
+SIZES = [(30, 30, 30), (31, 30, 30), (43, 43, 43), (44, 44, 44), (64, 64, 31), (64, 64, 32), (59, 59, 59), (61, 61, 61),
+         (131, 67, 61), (129, 130, 131)]
 
 
 @pytest.mark.parametrize("n", SIZES, ids=lambda n: "x".join(map(str, n)))
