@@ -39,11 +39,11 @@ namespace {
 enum Phase { PHASE_PRE = 0, PHASE_POST = 1, PHASE_AA_PENDING = 2, PHASE_AA_SWAPPED = 3 };
 
 // The share of a two-step launch's lanes and planes that must be the domain's
-// own for it to be taken.  Single steps / pairs, us per step, BGK (MRT):
-//   FP64  96^3 (0.52) 46 / 48 (46 / 52)   112^3 (0.66) 84 / 70 (83 / 75)
-//        130^3 (0.54) 130 / 127 (129 / 138)   256^3 (0.90) 983 / 630 (988 / 680)
-//   FP32  80^3 (0.34) 18 / 18 (17 / 19)   96^3 28 / 21   130^3 65 / 63   256^3 484 / 290
-constexpr double PAIR_FILL_F64 = 0.6, PAIR_FILL_F32 = 0.5;
+// own for it to be taken.  Single steps / pairs, us per step, BGK, couette:
+//   FP64  80^3 (0.34) 26 / 31   97^3 (0.48) 54 / 47   130^3 (0.54) 131 / 124
+//         112^3 (0.66) 86 / 66   256^3 (0.90) 983 / 660
+//   FP32  64^3 (0.31) 9.8 / 8.5   80^3 17.5 / 17.0   130^3 64 / 64   256^3 487 / 279
+constexpr double PAIR_FILL_F64 = 0.45, PAIR_FILL_F32 = 0.3;
 
 size_t elem_size(int storage) { return storage == HLBM_F64 ? 8 : (storage == HLBM_F32 ? 4 : 2); }
 

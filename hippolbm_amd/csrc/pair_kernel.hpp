@@ -15,20 +15,20 @@
 //   c_z =  0 of plane s - 1   written in the iteration before,
 //   c_z = +1 of plane s - 2   kept in registers for an iteration, then written,
 // so each of the 16 directions that leave the column needs one buffer only, and
-// the three that stay in it (rest, +z, -z) need none.  FP32 has room for more:
-// two sets of buffers, used in turn, which leaves one barrier per plane, and
+// the three that stay in it (rest, +z, -z) need none.  FP32 has room for
+// more: two sets of buffers, used in turn, which leaves one barrier per plane, and
 // registers for the next plane's loads, issued before step two.  (In FP64 those
 // loads spill: 512^3 4.7 ms per step without them, 8.9 ms with.)
 //
 // A node whose upstream neighbour is outside a non-periodic face pushes its own
-// opposite population (plus the moving-wall term) into the slot it will pull
-// from; that slot belongs to a node outside the domain, which nobody else
-// writes.  The arithmetic per node and step is the single step's own code, so
-// populations are the same bit for bit.
+// opposite population into the slot it will pull from; that slot belongs to a
+// node outside the domain, which nobody else writes.  The arithmetic per node and
+// step is the single step's own code, so the result is the same bit for bit.
 //
 // Taken by domains without walls, boundary programs and start_iteration boxes,
-// in FP64 and FP32 storage (16-bit storage rounds between the steps and is near
-// its issue limit).
+// in FP64 and FP32.  16-bit storage would round between the steps; it is near
+// its issue limit already, and the second stepping of the ring and the rounding
+// made 512^3 FP16 2.18 ms per step instead of 2.05 (200^3 171 us instead of 124).
 #pragma once
 
 #include "step_kernel.hpp"
@@ -85,9 +85,10 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
   using O = StoreOps<S>;
   using C = typename O::C;
   constexpr int TY = PAIR_TY, R = TY + 2, W = PAIR_TX + 2;
-  constexpr bool AHEAD = sizeof(S) == 4;    // the next plane's loads before step two
+  static_assert(std::is_same<S, C>::value, "populations pass between the steps as they are stored");
+  constexpr bool AHEAD = sizeof(S) == 4;  // the next plane's loads before step two
   constexpr int BUFS = sizeof(S) == 4 ? 2 : 1;
-  __shared__ C buf[BUFS][16][R][W];
+  __shared__ S buf[BUFS][16][R][W];
 
   // tiles next to each other in y run on the same XCD at the same time: they
   // share the rows between them
@@ -127,6 +128,14 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
   // the node's neighbours outside a non-periodic face
   const bool fxm = !px && x == 0, fxp = !px && x == nx - 1, fym = !py && y == 0, fyp = !py && y == ny - 1;
   const bool wave_face = __any(act && (fxm || fxp || fym || fyp));
+  // direction i's upstream node is outside (zout: outside a z face)
+  auto outside = [&](auto ic, bool zout) {
+    constexpr int i = decltype(ic)::value;
+    bool o = zout;
+    if constexpr (CX(i) != 0) o = o || (CX(i) == 1 ? fxm : fxp);
+    if constexpr (CY(i) != 0) o = o || (CY(i) == 1 ? fym : fyp);
+    return o;
+  };
 
   // byte offsets inside a plane: of the rows and columns populations come from,
   // added where they are used (nine sums kept across the loop would spill)
@@ -142,37 +151,24 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
   auto plane_valid = [&](int s) { return pz || (s >= 0 && s < nz); };
   auto wrapped = [&](int s) { return s < 0 ? s + nz : (s >= nz ? s - nz : s); };
 
-  // direction i's upstream node is outside a non-periodic face (zout: a z face)
-  auto outside = [&](auto ic, bool zout) {
-    constexpr int i = decltype(ic)::value;
-    bool o = zout;
-    if constexpr (CX(i) != 0) o = o || (CX(i) == 1 ? fxm : fxp);
-    if constexpr (CY(i) != 0) o = o || (CY(i) == 1 ? fym : fyp);
-    return o;
-  };
-  // step one's populations arriving at the node in plane s
-  auto gather = [&](int s, C* f) {
+  // step one's populations arriving at the node in plane s, as stored
+  auto gather = [&](int s, S* f) {
     const int z = wrapped(s);
-    if (!pz && (z == 0 || z == nz - 1)) {
-      const NodeNbrs a = node_nbrs<S>(p, x, y, z);
-      gather_select<S, MODE_FUSED>(p, (uint32_t)z * nxy * (uint32_t)sizeof(S) + off(1, 1), a, 0u, f);
-    } else if (wave_face) {
+    const bool zlo = !pz && z == 0, zhi = !pz && z == nz - 1;
+    if (wave_face || zlo || zhi) {
       // as gather_select: a lane whose upstream node is outside takes its own
       // opposite population, both addressed from the first plane of the pair
-      const uint32_t stb = (uint32_t)(p.stride * sizeof(S)), pb = nxy * (uint32_t)sizeof(S);
+      const uint32_t stb = (uint32_t)(p.stride * sizeof(S)), pb = nxy * unit;
       const uint32_t zo[3] = {(uint32_t)wrapped(z - 1) * pb, (uint32_t)z * pb, (uint32_t)wrapped(z + 1) * pb};
-      f[0] = O::ld(at_bytes(scalar_ptr(fin), lane_offset(off(1, 1) + zo[1])), 0);
+      f[0] = *at_bytes(scalar_ptr(fin), lane_offset(off(1, 1) + zo[1]));
       const S* b = fin;
       static_for<1, Q>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         constexpr int lo = (i & 1) ? i : i - 1;
         if constexpr (i & 1) b = scalar_ptr(b + (size_t)(i == 1 ? 1 : 2) * p.stride);
-        uint32_t o = off(1 - CY(i), 1 - CX(i)) + ((uint32_t)(i - lo) * stb + zo[1 - CZ(i)]);
-        if constexpr (CX(i) != 0 || CY(i) != 0) {
-          const uint32_t own = off(1, 1) + ((uint32_t)(OPP(i) - lo) * stb + zo[1]);
-          o = outside(ic, false) ? own : o;
-        }
-        f[i] = O::ld(at_bytes(b, o), 0);
+        const uint32_t pull = off(1 - CY(i), 1 - CX(i)) + ((uint32_t)(i - lo) * stb + zo[1 - CZ(i)]);
+        const uint32_t own = off(1, 1) + ((uint32_t)(OPP(i) - lo) * stb + zo[1]);
+        f[i] = *at_bytes(b, outside(ic, CZ(i) == 1 ? zlo : (CZ(i) == -1 ? zhi : false)) ? own : pull);
       });
     } else {
       const size_t zo[3] = {(size_t)wrapped(z - 1) * nxy, (size_t)z * nxy, (size_t)wrapped(z + 1) * nxy};
@@ -181,40 +177,41 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
         constexpr int i = decltype(ic)::value;
         b = scalar_ptr(i ? b + p.stride : b);
         const S* q = scalar_ptr(b + zo[1 - CZ(i)]);
-        f[i] = O::ld(at_bytes(q, lane_offset(off(1 - CY(i), 1 - CX(i)))), 0);
+        f[i] = *at_bytes(q, lane_offset(off(1 - CY(i), 1 - CX(i))));
       });
     }
   };
-  auto wall_term = [&](auto ic, bool zout) -> C {
-    constexpr int i = decltype(ic)::value;
-    if constexpr (CZ(i) == 0) {
-      return C(0);
-    } else {
-      constexpr int sd = CZ(i) == 1 ? 0 : 1;
-      return zout && p.cav_gather && p.cav_on[sd] ? cav_coef<C>(p, sd, cavity_slot(i)) : C(0);
-    }
+  // the moving-wall terms of the populations that bounced off a z face
+  auto add_wall = [&](int z, C* f) {
+    if (pz || !p.cav_gather) return;
+    static_for<0, 2>([&](auto sc) {
+      constexpr int sd = decltype(sc)::value;
+      if (p.cav_on[sd] && z == (sd ? nz - 1 : 0))
+        static_for<1, Q>([&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          if constexpr (CZ(i) == (sd ? -1 : 1)) f[i] += cav_coef<C>(p, sd, cavity_slot(i));
+        });
+    });
   };
-
-  C gn[Q];              // arriving in plane s
-  C up[4] = {}, h0 = C(0), h5 = C(0), u5 = C(0);  // kept: c_z = +1 and rest of plane s - 1, +z of plane s - 2
+  S gn[Q];  // arriving in plane s
+  // kept, as stored: c_z = +1 diagonals and rest of plane s - 1; +z of planes s - 1 and s - 2
+  S up[4] = {}, h0 = {}, h5 = {}, u5 = {};
   if (AHEAD && act && plane_valid(zs - 1)) gather(zs - 1, gn);
   for (int s = zs - 1; s <= ze; s++) {
     const bool valid = plane_valid(s), before = plane_valid(s - 1);
     auto& lds = buf[BUFS == 2 ? s & 1 : 0];
     auto& next = buf[BUFS == 2 ? ~s & 1 : 0];  // read by the next iteration
-    C f[Q];
-    if constexpr (AHEAD) {
-#pragma unroll
-      for (int i = 0; i < Q; i++) f[i] = gn[i];
-    } else {
-      if (act && valid) gather(s, f);
-    }
+    S h[Q];  // step one's populations of plane s
     if (act && valid) {
-      collide_node<S, COLL, MODE_FUSED, false, false>(p, 0u, false, f);
+      if constexpr (!AHEAD) gather(s, gn);
+#pragma unroll
+      for (int i = 0; i < Q; i++) h[i] = gn[i];
+      add_wall(wrapped(s), h);
+      collide_node<S, COLL, MODE_FUSED, false, false>(p, 0u, false, h);
       // these reach step two in registers, rounded as the others are by LDS
-      f[0] = rounded(f[0]);
-      f[5] = rounded(f[5]);
-      f[6] = rounded(f[6]);
+      h[0] = rounded(h[0]);
+      h[5] = rounded(h[5]);
+      h[6] = rounded(h[6]);
     }
     if (AHEAD && s < ze && act && plane_valid(s + 1)) gather(s + 1, gn);
 
@@ -222,7 +219,7 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
     if (act && valid) {
       static_for<1, Q>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        if constexpr (CZ(i) == -1 && pair_slot(i) >= 0) lds[pair_slot(i)][r][c] = f[i];
+        if constexpr (CZ(i) == -1 && pair_slot(i) >= 0) lds[pair_slot(i)][r][c] = h[i];
       });
     }
     const bool top = !pz && s == nz;  // plane s - 1 lies on the high z face
@@ -230,7 +227,7 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
       static_for<1, Q>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         if constexpr (CZ(i) == -1 && pair_slot(i) >= 0) {
-          if (outside(ic, top)) lds[pair_slot(i)][r - CY(i)][c - CX(i)] = up[pair_slot(OPP(i)) - 8] + wall_term(ic, top);
+          if (outside(ic, top)) lds[pair_slot(i)][r - CY(i)][c - CX(i)] = up[pair_slot(OPP(i)) - 8];
         }
       });
     }
@@ -239,22 +236,22 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
     // step two: plane s - 1
     if (s > zs && mine) {
       const int z = s - 1;
-      C f2[Q];
-      f2[0] = h0;
-      f2[5] = u5;
-      f2[6] = top ? h5 + wall_term(std::integral_constant<int, 6>{}, true) : f[6];
+      C f[Q];
+      f[0] = h0;
+      f[5] = u5;
+      f[6] = top ? h5 : h[6];
       static_for<1, Q>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        if constexpr (pair_slot(i) >= 0) f2[i] = lds[pair_slot(i)][r - CY(i)][c - CX(i)];
+        if constexpr (pair_slot(i) >= 0) f[i] = lds[pair_slot(i)][r - CY(i)][c - CX(i)];
       });
-      const uint32_t idx = (uint32_t)z * nxy + off(1, 1) / (uint32_t)sizeof(S);
-      collide_node<S, COLL, MODE_FUSED>(p, idx, false, f2);
+      add_wall(z, f);
+      collide_node<S, COLL, MODE_FUSED>(p, (uint32_t)z * nxy + off(1, 1) / unit, false, f);
       S* b = (S*)p.fout + (size_t)z * nxy;
       const uint32_t bo = lane_offset(off(1, 1));
       static_for([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         b = scalar_ptr(i ? b + p.stride : b);
-        O::st(at_bytes(b, bo), 0, f2[i]);
+        O::st(at_bytes(b, bo), 0, f[i]);
       });
     }
     if constexpr (BUFS == 1) lds_barrier();
@@ -265,7 +262,7 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
       static_for<1, Q>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         if constexpr (pair_slot(i) >= 0) {
-          if (CZ(i) == 0 && valid) next[pair_slot(i)][r][c] = f[i];
+          if (CZ(i) == 0 && valid) next[pair_slot(i)][r][c] = h[i];
           if (CZ(i) == 1 && before) next[pair_slot(i)][r][c] = up[pair_slot(i) - 8];
         }
       });
@@ -274,17 +271,16 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
       static_for<1, Q>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         if constexpr (pair_slot(i) >= 0 && CZ(i) >= 0) {
-          const bool zout = CZ(i) == 1 && bottom;
-          if (outside(ic, zout)) next[pair_slot(i)][r - CY(i)][c - CX(i)] = f[OPP(i)] + wall_term(ic, zout);
+          if (outside(ic, CZ(i) == 1 && bottom)) next[pair_slot(i)][r - CY(i)][c - CX(i)] = h[OPP(i)];
         }
       });
     }
-    u5 = bottom ? f[6] + wall_term(std::integral_constant<int, 5>{}, true) : h5;
-    h5 = f[5];
-    h0 = f[0];
+    u5 = bottom ? h[6] : h5;
+    h5 = h[5];
+    h0 = h[0];
     static_for<1, Q>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
-      if constexpr (CZ(i) == 1 && pair_slot(i) >= 0) up[pair_slot(i) - 8] = f[i];
+      if constexpr (CZ(i) == 1 && pair_slot(i) >= 0) up[pair_slot(i) - 8] = h[i];
     });
   }
 }

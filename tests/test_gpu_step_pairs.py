@@ -2,8 +2,9 @@
 
 HLBM_PAIRS=2 takes the two-step kernel at every size, HLBM_PAIRS=0 never.  The
 node's arithmetic is the same code, so every population must be equal bit for
-bit: FP64 against the oracle, FP32 against single steps.  Sizes around the tile
-(64 columns, 9 or 12 rows) and the segment, with rings that wrap onto the tile
+bit: FP64 against the oracle, the reduced storages (of which FP32 has the
+kernel) against single steps.  Sizes around the tile
+(64 columns, 13 rows) and the segment, with rings that wrap onto the tile
 itself, faces on every axis and their edges and corners (the moving wall
 included), odd and even step counts, rho and u of the last step."""
 import numpy as np
@@ -15,8 +16,8 @@ from hippolbm_amd.engine import W, Simulation
 
 pytestmark = pytest.mark.gpu
 
-# one tile and less; exactly one, one more; rows 9 / 12 and their neighbours; 64 and 128 planes and their neighbours
-SIZES = [(2, 2, 2), (5, 3, 4), (64, 9, 6), (65, 10, 5), (63, 12, 7), (128, 13, 3), (130, 25, 9), (20, 7, 64), (17, 5, 66),
+# one tile and less; exactly one, one more; 12, 13 and 26 rows; several segments
+SIZES = [(2, 2, 2), (5, 3, 4), (64, 9, 6), (65, 10, 5), (63, 12, 7), (128, 13, 3), (130, 26, 9), (20, 7, 64), (17, 5, 66),
          (9, 11, 130)]
 
 
@@ -74,11 +75,12 @@ def test_pairs_equal_single_steps(n, periodic, collision, monkeypatch):
     assert np.array_equal(rho, last[0]) and np.array_equal(u, last[1])
     assert np.array_equal(f, one.dom.get_f())
     one.dom.close()
-    runs = []
-    for pairs in (2, 0):
-        s = start(d, n, "f32", monkeypatch, pairs, f0)
-        s.run(8)
-        runs.append((s.dom.get_f(),) + s.dom.get_macro())
-        s.dom.close()
-    for a, b in zip(*runs):
-        assert np.array_equal(a, b)
+    for storage in ("f32", "f16", "bf16"):
+        runs = []
+        for pairs in (2, 0):
+            s = start(d, n, storage, monkeypatch, pairs, f0)
+            s.run(8)
+            runs.append((s.dom.get_f(),) + s.dom.get_macro())
+            s.dom.close()
+        for a, b in zip(*runs):
+            assert np.array_equal(a, b), storage
