@@ -67,6 +67,15 @@ inline PairGrid pair_grid(int nx, int ny, int nz, int64_t* cost) {
   return g;
 }
 
+// FP64: from this size of the two lattices together the new populations are
+// stored with the non-temporal hint, so that the planes neighbouring tiles still
+// share stay in L2.  Up to it the Infinity Cache (256 MiB) holds much of what was
+// stored until the next pass reads it.  Without / with the hint, us per step, BGK:
+// 80^3 29.9 / 30.8   96^3 (257 MiB) 38.0 / 40.6   104^3 (326) 52.8 / 51.6
+// 112^3 66 / 59   200^3 374 / 325   512^3 4500-4890 / 4290-4700.
+// (FP32 without the hint: no difference at any size.)
+constexpr int64_t PAIR_STREAM_BYTES = 320ll << 20;
+
 // LDS slot of a direction that leaves its column, in the order c_z = 0, +1, -1.
 HLBM_HD constexpr int pair_slot(int i) {
   constexpr int s[Q] = {-1, 0, 1, 2, 3, -1, -1, 4, 5, 6, 7, 8, 12, 13, 9, 10, 14, 15, 11};
@@ -80,7 +89,7 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <class S, int COLL>
+template <class S, int COLL, bool STREAM>
 __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepParams p, const PairGrid g) {
   using O = StoreOps<S>;
   using C = typename O::C;
@@ -253,7 +262,10 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
       static_for([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         b = scalar_ptr(i ? b + p.stride : b);
-        O::st(at_bytes(b, bo), 0, f[i]);
+        if constexpr (STREAM)
+          __builtin_nontemporal_store(f[i], at_bytes(b, bo));
+        else
+          *at_bytes(b, bo) = f[i];
       });
     }
     if constexpr (BUFS == 1) lds_barrier();

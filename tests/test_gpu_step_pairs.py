@@ -84,3 +84,20 @@ def test_pairs_equal_single_steps(n, periodic, collision, monkeypatch):
             s.dom.close()
         for a, b in zip(*runs):
             assert np.array_equal(a, b), storage
+
+
+@pytest.mark.parametrize("n", [(130, 92, 92), (130, 92, 93), (257, 67, 65)], ids=lambda n: "x".join(map(str, n)))
+def test_pairs_above_the_cache(n, monkeypatch):
+    """FP64 below and above the 320 MiB from which the populations are stored
+    with the non-temporal hint: the largest size of the plain stores, the next
+    one and a ragged one, equal to single steps bit for bit."""
+    print("pairs above the cache", n, flush=True)
+    d = deck(n, (1, 0, 0), "bgk", 1e-4)
+    f0 = W.reshape(19, 1, 1, 1) * (1.0 + 1e-2 * np.random.default_rng(2).uniform(-1, 1, (19, n[2], n[1], n[0])))
+    runs = []
+    for pairs in (2, 0):
+        sim = start(d, n, "f64", monkeypatch, pairs, f0)
+        sim.run(5)
+        runs.append(sim.dom.get_f())
+        sim.dom.close()
+    assert np.array_equal(runs[0], runs[1])
