@@ -87,6 +87,7 @@ struct hlbm_domain {
   int xcd_remap = 1;
   int npt = 1;
   int force_wide = 0;
+  int linear = 1;   // consecutive nodes per workgroup on ragged grids: 0 never, 1 large domains, 2 any size
   int pairs = 1;    // two steps per pass where it applies: 0 never, 1 large domains, 2 any size
   int variant = 0;  // bulk-kernel variant (hlbm_set_launch)
   int boundary_first = 1;  // program-plane kernel before the bulk kernel (measured 1-2 % faster)
@@ -135,18 +136,33 @@ static unsigned tiles_y(const hlbm_domain* h) {
   return (along(h, 1) + rows - 1) / rows;
 }
 
-// Tiles of a ragged grid leave lanes without a node (151 x 150 in tiles of
-// 128 x 2: 41 % of them): from 2 % of such lanes on, workgroups take
-// consecutive nodes instead (one node per thread).  Measured: 201 x 173 x 119
-// MRT BF16 112 -> 61 us per step (21 % of the tile lanes idle, and issue-bound);
-// 151 x 150 x 149 AA FP32 82 us either way (bound by memory); grids without idle
-// lanes keep the tiles, whose coordinates cost less (512^3 FP16 the same within
-// 0.5 %).
+// Workgroups take consecutive nodes (one node per thread) instead of tiles where
+//  - 2 % of the tiles' lanes would have no node (151 x 150 in tiles of 128 x 2:
+//    41 % of them), or
+//  - rows are not whole cache lines: a row's waves then start inside one, and the
+//    lines that two waves write in part cost HBM a read.
+// Measured, us per step, tiles / consecutive:
+//   201 x 173 x 119 MRT BF16 112 / 67 (21 % idle); 151 x 150 x 149 AA FP32 82 / 82;
+//   380 x 260 x 200 (1 % idle) BGK FP16 462 / 305, FP32 822 / 613, FP64 1252 / 1174,
+//   AA FP32 652 / 622, spheres MRT BF16 571 / 341; 126 x 128 x 128 FP16 38.0 / 32.3.
+// Grids without either keep the tiles, whose coordinates cost less (512^3 FP16,
+// 96^3, 160^3: the same within 1 %).  So do small ones: partly written lines meet
+// in the caches there, and what remains is the idle lanes, against the latency of
+// fuller waves:
+//   idle lanes above 1/8 of the waves that have work:  24^3 FP32 BGK 3.9 / 4.3, 48 x 40 x 40 4.6 / 5.1;
+//     50^3 5.8 / 5.3, 72 x 64 x 64 BF16 AA 10.0 / 8.1
+//   below:  63 x 60 x 60 BF16 AA 6.6 / 7.1, 57 x 58 x 60 FP64 11.8 / 12.4;
+//     63 x 80 x 80 9.3 / 9.1, 21.5 / 21.6; 63 x 100 x 100 12.2 / 11.1, 31.5 / 30.4
+constexpr uint32_t LINEAR_MIN_IDLE = 100000, LINEAR_MIN_NODES = 350000;
 static bool linear_nodes(const hlbm_domain* h) {
-  if (eff_npt(h) != 1) return false;
-  const uint64_t gx = (along(h, 0) + h->block.x - 1) / h->block.x;
+  if (eff_npt(h) != 1 || !h->linear) return false;
+  const uint64_t gx = (along(h, 0) + h->block.x - 1) / h->block.x, N = h->N;
   const uint64_t lanes = gx * h->block.x * tiles_y(h) * h->block.y * along(h, 2);
-  return lanes * 50 > (uint64_t)h->N * 51;
+  if (h->linear == 1 && N < LINEAR_MIN_NODES) {
+    const uint64_t busy = ((uint64_t)along(h, 0) + 63) / 64 * 64 * along(h, 1) * along(h, 2);
+    return N >= LINEAR_MIN_IDLE && busy * 7 > N * 8;
+  }
+  return (uint64_t)along(h, 0) * h->esize % 128 != 0 || lanes * 50 > N * 51;
 }
 
 static dim3 grid_for(const hlbm_domain* h) {
@@ -507,6 +523,7 @@ int hlbm_domain_create(const hlbm_domain_desc* desc, hlbm_domain** out) {
   if (const char* np = getenv("HLBM_NPT")) h->npt = atoi(np) == 2 ? 2 : 1;
   // the 64-bit-address variant otherwise runs only on domains above 2^32 bytes per plane
   if (const char* fw = getenv("HLBM_FORCE_WIDE")) h->force_wide = atoi(fw) ? 1 : 0;
+  if (const char* li = getenv("HLBM_LINEAR")) h->linear = std::max(0, std::min(2, atoi(li)));
   if (const char* pr = getenv("HLBM_PAIRS")) h->pairs = std::max(0, std::min(2, atoi(pr)));
   if (const char* bf = getenv("HLBM_BOUNDARY_FIRST")) h->boundary_first = atoi(bf) ? 1 : 0;
   if (const char* ov = getenv("HLBM_OVERLAP")) h->overlap = atoi(ov) ? 1 : 0;

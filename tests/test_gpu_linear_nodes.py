@@ -62,3 +62,18 @@ def test_rows_that_do_not_fill_tiles(n, how):
         sim.run(steps)
         assert np.array_equal(sim.dom.get_f(), ref.o.node_f())
     sim.dom.close()
+
+
+# the last four: under 2 % of the tiles' lanes without a node, taken for rows that are not whole cache lines
+@pytest.mark.parametrize("n", SIZES + [(127, 4, 3), (126, 8, 2), (255, 4, 2), (510, 2, 3)],
+                         ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("how", ["ab", "aa", "wide", "yzx"])
+def test_consecutive_nodes_at_any_size(n, how, monkeypatch):
+    """HLBM_LINEAR=2: also below the sizes from which the rule takes them."""
+    monkeypatch.setenv("HLBM_LINEAR", "2")
+    test_rows_that_do_not_fill_tiles(n, how)
+
+
+@pytest.mark.parametrize("n", [(47, 48, 44), (47, 48, 45), (63, 74, 75), (63, 75, 76)], ids=lambda n: "x".join(map(str, n)))
+def test_the_sizes_from_which_nodes_are_consecutive(n):
+    test_rows_that_do_not_fill_tiles(n, "ab")
