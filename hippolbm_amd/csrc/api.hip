@@ -43,7 +43,8 @@ enum Phase { PHASE_PRE = 0, PHASE_POST = 1, PHASE_AA_PENDING = 2, PHASE_AA_SWAPP
 //   FP64  80^3 (0.34) 26 / 31   97^3 (0.48) 54 / 47   130^3 (0.54) 131 / 124
 //         112^3 (0.66) 86 / 66   256^3 (0.90) 983 / 660
 //   FP32  64^3 (0.31) 9.8 / 8.5   80^3 17.5 / 17.0   130^3 64 / 64   256^3 487 / 279
-constexpr double PAIR_FILL_F64 = 0.45, PAIR_FILL_F32 = 0.3;
+//   16-bit (BGK, rows of whole half lines)  128^3 (0.76) 34 / 34   256^3 (0.90) 252 / 236
+constexpr double PAIR_FILL_F64 = 0.45, PAIR_FILL_F32 = 0.3, PAIR_FILL_16 = 0.87;
 
 size_t elem_size(int storage) { return storage == HLBM_F64 ? 8 : (storage == HLBM_F32 ? 4 : 2); }
 
@@ -179,6 +180,9 @@ static RestShift dom_shift(const hlbm_domain* h) {
   return rest_shift(h->d.collision == HLBM_MRT, h->d.mrt_custom, h->d.mrt_rates);
 }
 
+// The rounding seed of time step t.
+static uint32_t step_seed(int64_t t) { return mix32((uint32_t)t * 0x9E3779B9u + 1u); }
+
 static StepParams base_params(hlbm_domain* h) {
   StepParams p = h->plan;
   p.nx = h->nx;
@@ -228,7 +232,7 @@ static StepParams base_params(hlbm_domain* h) {
   p.pair32 = ((uint64_t)h->stride + h->N) * h->esize < 0xFFFFFFFFull ? 1 : 0;
   // 16-bit storage: stochastic rounding keyed on (node, time step)
   p.sr = (h->d.storage == HLBM_F16 || h->d.storage == HLBM_BF16) && !h->d.round_nearest ? 1 : 0;
-  p.seed = mix32((uint32_t)h->t * 0x9E3779B9u + 1u);
+  p.seed = step_seed(h->t);
   return p;
 }
 
@@ -420,21 +424,25 @@ static int launch(hlbm_domain* h, int mode, bool write_macro, hipStream_t s, voi
 // pull, collide, store, and large enough to fill the chip with its tiles.
 static bool steps_in_pairs(const hlbm_domain* h, const StepParams& p, PairGrid* g) {
   if (!h->pairs || h->d.pattern != HLBM_PATTERN_AB) return false;
-  if (h->d.storage != HLBM_F64 && h->d.storage != HLBM_F32) return false;
   if (h->any_wall || p.nprog || p.prog_planes || p.nset || p.nspec || !default_layout_p(h)) return false;
   if (!p.pair32 || wide_offsets(p, h->esize)) return false;
-  const double fill = h->d.storage == HLBM_F64 ? PAIR_FILL_F64 : PAIR_FILL_F32;
+  const bool narrow = h->esize == 2;
+  if (narrow && h->d.collision == HLBM_MRT) return false;
+  const double fill = h->d.storage == HLBM_F64 ? PAIR_FILL_F64 : (narrow ? PAIR_FILL_16 : PAIR_FILL_F32);
   int64_t cost;
   *g = pair_grid(h->nx, h->ny, h->nz, &cost);
+  if (h->pairs == 1 && narrow && h->nx % 32 != 0) return false;
   return h->pairs == 2 || (double)h->N >= fill * (double)cost * (PAIR_TX * PAIR_TY);
 }
 
-static int launch_pair(hlbm_domain* h, StepParams& p, const PairGrid& g, bool write_macro, hipStream_t s) {
+static int launch_pair(hlbm_domain* h, StepParams& p, PairGrid& g, bool write_macro, hipStream_t s) {
   p.fin = h->buf[h->cur];
   p.fout = h->buf[h->cur ^ 1];
   p.write_macro = write_macro ? 1 : 0;
   const int coll = h->d.collision == HLBM_MRT ? COLL_MRT : COLL_BGK;
-  const hipError_t e = h->d.storage == HLBM_F64 ? launch_pair_f64(coll, g, p, s) : launch_pair_f32(coll, g, p, s);
+  g.seed2 = step_seed(h->t + 1);
+  const hipError_t e = h->d.storage == HLBM_F64 ? launch_pair_f64(coll, g, p, s)
+                                                : launch_pair_lowp(h->d.storage, coll, g, p, s);
   if (e != hipSuccess) return fail(HLBM_ERR_HIP, std::string("step pair launch: ") + hipGetErrorString(e));
   h->cur ^= 1;
   return HLBM_OK;

@@ -126,23 +126,21 @@ hipError_t step_dispatch(int coll, int mode, int npt, dim3 grid, dim3 block, con
   return step_go_npt<S, COLL_MRT, MODE_COLLIDE>(npt, grid, block, p, s);
 }
 
-template <class S, bool STREAM>
-hipError_t pair_go_st(int coll, const PairGrid& g, const StepParams& p, hipStream_t s) {
+template <class S, int COLL, bool STREAM>
+hipError_t pair_go_st(const PairGrid& g, const StepParams& p, hipStream_t s) {
   const dim3 grid((unsigned)(g.tx * g.ty * g.segs)), block((PAIR_TY + 3) * 64);
-  if (coll == COLL_BGK)
-    hipLaunchKernelGGL((pair_kernel<S, COLL_BGK, STREAM>), grid, block, 0, s, p, g);
-  else
-    hipLaunchKernelGGL((pair_kernel<S, COLL_MRT, STREAM>), grid, block, 0, s, p, g);
+  hipLaunchKernelGGL((pair_kernel<S, COLL, STREAM>), grid, block, 0, s, p, g);
   return hipGetLastError();
 }
-template <class S>
-hipError_t pair_go(int coll, const PairGrid& g, const StepParams& p, hipStream_t s) {
+template <class S, int COLL>
+hipError_t pair_go(const PairGrid& g, const StepParams& p, hipStream_t s) {
   if constexpr (sizeof(S) == 8)
-    if (2 * Q * (int64_t)sizeof(S) * p.nx * p.ny * p.nz <= PAIR_STREAM_BYTES) return pair_go_st<S, false>(coll, g, p, s);
-  return pair_go_st<S, true>(coll, g, p, s);
+    if (2 * Q * (int64_t)sizeof(S) * p.nx * p.ny * p.nz <= PAIR_STREAM_BYTES)
+      return pair_go_st<S, COLL, false>(g, p, s);
+  return pair_go_st<S, COLL, true>(g, p, s);
 }
 hipError_t launch_pair_f64(int coll, const PairGrid& g, const StepParams& p, hipStream_t s);
-hipError_t launch_pair_f32(int coll, const PairGrid& g, const StepParams& p, hipStream_t s);
+hipError_t launch_pair_lowp(int storage, int coll, const PairGrid& g, const StepParams& p, hipStream_t s);
 
 // FP64 storage, FP64 compute, no contraction (step_f64.hip)
 hipError_t launch_step_f64(int coll, int mode, int npt, dim3 grid, dim3 block, const StepParams& p, hipStream_t s);

@@ -15,20 +15,26 @@
 //   c_z =  0 of plane s - 1   written in the iteration before,
 //   c_z = +1 of plane s - 2   kept in registers for an iteration, then written,
 // so each of the 16 directions that leave the column needs one buffer only, and
-// the three that stay in it (rest, +z, -z) need none.  FP32 has room for
-// more: two sets of buffers, used in turn, which leaves one barrier per plane, and
+// the three that stay in it (rest, +z, -z) need none.  Below FP64 there is room
+// for more: two sets of buffers, used in turn, which leaves one barrier per plane, and
 // registers for the next plane's loads, issued before step two.  (In FP64 those
 // loads spill: 512^3 4.4 ms per step without them, 8.9 ms with.)
 //
 // A node whose upstream neighbour is outside a non-periodic face pushes its own
 // opposite population into the slot it will pull from; that slot belongs to a
-// node outside the domain, which nobody else writes.  The arithmetic per node and
-// step is the single step's own code, so the result is the same bit for bit.
+// node outside the domain, which nobody else writes.  Populations travel as they
+// are stored (16-bit storage: rounded with the first step's random words), and
+// the arithmetic per node and step is the single step's own code, so the result
+// is the same bit for bit.
 //
-// Taken by domains without walls, boundary programs and start_iteration boxes,
-// in FP64 and FP32.  16-bit storage would round between the steps; it is near
-// its issue limit already, and the second stepping of the ring and the rounding
-// made 512^3 FP16 2.18 ms per step instead of 2.05 (200^3 171 us instead of 124).
+// Taken by domains without walls, boundary programs and start_iteration boxes, MRT
+// only in FP64 and FP32.  Single / two steps per pass, ms per step: 512^3 BGK FP64
+// 7.3 / 4.4, 512 x 256 x 256 FP32 0.94 / 0.58 (5.1 TB/s of actual traffic: the
+// memory's limit for this pattern), 512^3 FP16 2.12 / 1.91, BF16 2.14 / 1.79.  A
+// plane of a 16-bit tile takes 5.6 us, 2.8 of them vector issue: half the bytes
+// leave the chain load, collide, LDS, collide in view, MRT (FP16 2.08 / 2.10)
+// lengthens it, and rows that end inside a cache line (500 x 400 x 200 586 / 664
+// us) meet stores of partial lines.
 #pragma once
 
 #include "step_kernel.hpp"
@@ -44,6 +50,7 @@ constexpr int PAIR_TY = 13;
 struct PairGrid {
   int32_t tx, ty, segs;  // tiles along x and y, segments along z
   int32_t planes;        // planes per segment
+  uint32_t seed2;        // rounding seed of the second step (StepParams::seed is the first's)
 };
 
 // The segments that cost the fewest planes: a CU holds one workgroup at a time
@@ -52,7 +59,7 @@ struct PairGrid {
 // against nx * ny * nz / (64 * 13) for a grid that fills it exactly.
 constexpr int PAIR_CUS = 256;
 inline PairGrid pair_grid(int nx, int ny, int nz, int64_t* cost) {
-  PairGrid g{(nx + PAIR_TX - 1) / PAIR_TX, (ny + PAIR_TY - 1) / PAIR_TY, 1, nz};
+  PairGrid g{(nx + PAIR_TX - 1) / PAIR_TX, (ny + PAIR_TY - 1) / PAIR_TY, 1, nz, 0u};
   *cost = INT64_MAX;
   for (int k = 1; k <= nz; k++) {
     const int planes = (nz + k - 1) / k, segs = (nz + planes - 1) / planes;
@@ -76,6 +83,12 @@ inline PairGrid pair_grid(int nx, int ny, int nz, int64_t* cost) {
 // (FP32 without the hint: no difference at any size.)
 constexpr int64_t PAIR_STREAM_BYTES = 320ll << 20;
 
+// What Rounder reads of a step's parameters.
+struct PairRounding {
+  int32_t sr;
+  uint32_t seed;
+};
+
 // LDS slot of a direction that leaves its column, in the order c_z = 0, +1, -1.
 HLBM_HD constexpr int pair_slot(int i) {
   constexpr int s[Q] = {-1, 0, 1, 2, 3, -1, -1, 4, 5, 6, 7, 8, 12, 13, 9, 10, 14, 15, 11};
@@ -94,9 +107,10 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
   using O = StoreOps<S>;
   using C = typename O::C;
   constexpr int TY = PAIR_TY, R = TY + 2, W = PAIR_TX + 2;
-  static_assert(std::is_same<S, C>::value, "populations pass between the steps as they are stored");
-  constexpr bool AHEAD = sizeof(S) == 4;  // the next plane's loads before step two
-  constexpr int BUFS = sizeof(S) == 4 ? 2 : 1;
+  constexpr bool AHEAD = sizeof(S) <= 4;  // the next plane's loads before step two
+  constexpr int BUFS = sizeof(S) <= 4 ? 2 : 1;
+  using Raw = std::conditional_t<sizeof(S) == 2, uint16_t, C>;
+  constexpr bool RAW = raw_store<S, COLL, MODE_FUSED>();
   __shared__ S buf[BUFS][16][R][W];
 
   // Tiles next to each other in x run on the same XCD at the same time: a ring's
@@ -204,6 +218,19 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
         });
     });
   };
+  // populations as a step stores them (16-bit: rounded with that step's words)
+  auto stored = [&](uint32_t seed, int z, const C* f, S* h) {
+    const PairRounding rp{p.sr, seed};
+    const Rounder<S> rw(rp, (uint32_t)z * nxy + (uint32_t)y * (uint32_t)nx + (uint32_t)x);
+    static_for([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      if constexpr (RAW)
+        h[i] = O::pack_sr_scaled(f[i], rw.word(i));
+      else
+        h[i] = O::pack_sr(f[i], rw.word(i));
+    });
+  };
+
   S gn[Q];  // arriving in plane s
   // kept, as stored: c_z = +1 diagonals and rest of plane s - 1; +z of planes s - 1 and s - 2
   S up[4] = {}, h0 = {}, h5 = {}, u5 = {};
@@ -215,14 +242,18 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
     S h[Q];  // step one's populations of plane s
     if (act && valid) {
       if constexpr (!AHEAD) gather(s, gn);
+      C f[Q];
 #pragma unroll
-      for (int i = 0; i < Q; i++) h[i] = gn[i];
-      add_wall(wrapped(s), h);
-      collide_node<S, COLL, MODE_FUSED, false, false>(p, 0u, false, h);
+      for (int i = 0; i < Q; i++) f[i] = O::unpack(gn[i]);
+      add_wall(wrapped(s), f);
+      collide_node<S, COLL, MODE_FUSED, RAW, false>(p, 0u, false, f);
+      stored(p.seed, wrapped(s), f, h);
       // these reach step two in registers, rounded as the others are by LDS
-      h[0] = rounded(h[0]);
-      h[5] = rounded(h[5]);
-      h[6] = rounded(h[6]);
+      if constexpr (!O::narrow16) {
+        h[0] = rounded(h[0]);
+        h[5] = rounded(h[5]);
+        h[6] = rounded(h[6]);
+      }
     }
     if (AHEAD && s < ze && act && plane_valid(s + 1)) gather(s + 1, gn);
 
@@ -248,24 +279,26 @@ __global__ void __launch_bounds__((PAIR_TY + 3) * 64) pair_kernel(const StepPara
     if (s > zs && mine) {
       const int z = s - 1;
       C f[Q];
-      f[0] = h0;
-      f[5] = u5;
-      f[6] = top ? h5 : h[6];
+      f[0] = O::unpack(h0);
+      f[5] = O::unpack(u5);
+      f[6] = O::unpack(top ? h5 : h[6]);
       static_for<1, Q>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        if constexpr (pair_slot(i) >= 0) f[i] = lds[pair_slot(i)][r - CY(i)][c - CX(i)];
+        if constexpr (pair_slot(i) >= 0) f[i] = O::unpack(lds[pair_slot(i)][r - CY(i)][c - CX(i)]);
       });
       add_wall(z, f);
-      collide_node<S, COLL, MODE_FUSED>(p, (uint32_t)z * nxy + off(1, 1) / unit, false, f);
+      collide_node<S, COLL, MODE_FUSED, RAW>(p, (uint32_t)z * nxy + off(1, 1) / unit, false, f);
+      S o[Q];
+      stored(g.seed2, z, f, o);
       S* b = (S*)p.fout + (size_t)z * nxy;
       const uint32_t bo = lane_offset(off(1, 1));
       static_for([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         b = scalar_ptr(i ? b + p.stride : b);
         if constexpr (STREAM)
-          __builtin_nontemporal_store(f[i], at_bytes(b, bo));
+          __builtin_nontemporal_store(__builtin_bit_cast(Raw, o[i]), (Raw*)at_bytes(b, bo));
         else
-          *at_bytes(b, bo) = f[i];
+          *at_bytes(b, bo) = o[i];
       });
     }
     if constexpr (BUFS == 1) lds_barrier();

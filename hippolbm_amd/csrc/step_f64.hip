@@ -10,7 +10,7 @@ hipError_t launch_step_f64(int coll, int mode, int npt, dim3 grid, dim3 block, c
 }
 
 hipError_t launch_pair_f64(int coll, const PairGrid& g, const StepParams& p, hipStream_t s) {
-  return pair_go<double>(coll, g, p, s);
+  return coll == COLL_BGK ? pair_go<double, COLL_BGK>(g, p, s) : pair_go<double, COLL_MRT>(g, p, s);
 }
 
 hipError_t launch_batch_f64(int coll, unsigned blocks, const BatchParams& bp, hipStream_t s) {

@@ -153,6 +153,8 @@ struct StoreOps<double> {
   using C = double;
   static constexpr bool shifted = false;
   static constexpr bool narrow16 = false;
+  static __device__ __forceinline__ C unpack(double v) { return v; }
+  static __device__ __forceinline__ double pack_sr(C v, uint32_t) { return v; }
   static __device__ __forceinline__ C ld(const double* p, size_t i) { return p[i]; }
   static __device__ __forceinline__ void st(double* p, size_t i, C v) { p[i] = v; }
   static __device__ __forceinline__ void st_sr(double* p, size_t i, C v, uint32_t) { p[i] = v; }
@@ -165,6 +167,8 @@ struct StoreOps<float> {
   using C = float;
   static constexpr bool shifted = true;
   static constexpr bool narrow16 = false;
+  static __device__ __forceinline__ C unpack(float v) { return v; }
+  static __device__ __forceinline__ float pack_sr(C v, uint32_t) { return v; }
   static __device__ __forceinline__ C ld(const float* p, size_t i) { return p[i]; }
   static __device__ __forceinline__ void st(float* p, size_t i, C v) { __builtin_nontemporal_store(v, p + i); }
   static __device__ __forceinline__ void st_sr(float* p, size_t i, C v, uint32_t) {
@@ -179,26 +183,31 @@ struct StoreOps<_Float16> {
   static constexpr float SCALE = 8192.0f, INV_SCALE = 1.0f / 8192.0f;  // 2^13, 2^-13
   // fma(h, 2^-13, +0) is h * 2^-13 (exact) except that -0 loads as +0, and it
   // is one v_fma_mix_f32 (conversion and scaling together) instead of two
-  static __device__ __forceinline__ C ld(const _Float16* p, size_t i) {
-    return __builtin_fmaf((float)p[i], INV_SCALE, 0.0f);
-  }
+  static __device__ __forceinline__ C unpack(_Float16 h) { return __builtin_fmaf((float)h, INV_SCALE, 0.0f); }
+  static __device__ __forceinline__ C ld(const _Float16* p, size_t i) { return unpack(p[i]); }
   static __device__ __forceinline__ void st(_Float16* p, size_t i, C v) {
     __builtin_nontemporal_store((_Float16)(v * SCALE), p + i);
   }
   static __device__ __forceinline__ void st_sr(_Float16* p, size_t i, C v, uint32_t r) {
+    __builtin_nontemporal_store(pack_sr(v, r), p + i);
+  }
+  static __device__ __forceinline__ _Float16 pack_sr(C v, uint32_t r) {
     // FP16 keeps 10 of FP32's 23 mantissa bits: the 13 dropped ones are dithered
     // with the top 13 bits of r, i.e. (bits(v) + (r >> 19)) & ~0x1FFF, then
     // converted; gfx950's v_cvt_sr_f16_f32 does exactly this in one instruction
-    st_sr_scaled(p, i, v * SCALE, r);
+    return pack_sr_scaled(v * SCALE, r);
   }
   // the same for a value already multiplied by SCALE (the FP32 BGK collision
   // can fold the scale into its constants).  The instruction keeps the upper
   // half of its destination, which is not stored: the scaled value's own
   // register serves, no zeroed one is needed.
-  static __device__ __forceinline__ void st_sr_scaled(_Float16* p, size_t i, C s, uint32_t r) {
+  static __device__ __forceinline__ _Float16 pack_sr_scaled(C s, uint32_t r) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
     const h2 h = __builtin_amdgcn_cvt_sr_f16_f32(__builtin_bit_cast(h2, s), s, r, false);
-    __builtin_nontemporal_store(h[0], p + i);
+    return h[0];
+  }
+  static __device__ __forceinline__ void st_sr_scaled(_Float16* p, size_t i, C s, uint32_t r) {
+    __builtin_nontemporal_store(pack_sr_scaled(s, r), p + i);
   }
 };
 template <>
@@ -206,20 +215,22 @@ struct StoreOps<bf16s> {
   using C = float;
   static constexpr bool shifted = true;
   static constexpr bool narrow16 = true;
-  static __device__ __forceinline__ C ld(const bf16s* p, size_t i) {
-    return __uint_as_float(((uint32_t)p[i].v) << 16);
-  }
+  static __device__ __forceinline__ C unpack(bf16s b) { return __uint_as_float(((uint32_t)b.v) << 16); }
+  static __device__ __forceinline__ C ld(const bf16s* p, size_t i) { return unpack(p[i]); }
   static __device__ __forceinline__ void st(bf16s* p, size_t i, C v) {
     uint32_t u = __float_as_uint(v);
     u += 0x7FFFu + ((u >> 16) & 1u);  // round to nearest even
     __builtin_nontemporal_store((uint16_t)(u >> 16), (uint16_t*)(p + i));
   }
   static __device__ __forceinline__ void st_sr(bf16s* p, size_t i, C v, uint32_t r) {
+    __builtin_nontemporal_store(pack_sr(v, r).v, (uint16_t*)(p + i));
+  }
+  static __device__ __forceinline__ bf16s pack_sr(C v, uint32_t r) {
     // the 16 dropped bits dithered with the top 16 bits of r, (bits(v) + (r >> 16)) >> 16:
     // gfx950's v_cvt_sr_bf16_f32
     typedef short s2 __attribute__((ext_vector_type(2)));
     const s2 b = __builtin_amdgcn_cvt_sr_bf16_f32(__builtin_bit_cast(s2, v), v, r, false);
-    __builtin_nontemporal_store((uint16_t)b[0], (uint16_t*)(p + i));
+    return bf16s{(uint16_t)b[0]};
   }
 };
 

@@ -18,8 +18,10 @@ hipError_t launch_step_lowp(int storage, int coll, int mode, int npt, dim3 grid,
   }
 }
 
-hipError_t launch_pair_f32(int coll, const PairGrid& g, const StepParams& p, hipStream_t s) {
-  return pair_go<float>(coll, g, p, s);
+hipError_t launch_pair_lowp(int storage, int coll, const PairGrid& g, const StepParams& p, hipStream_t s) {
+  if (storage == 1) return coll == COLL_BGK ? pair_go<float, COLL_BGK>(g, p, s) : pair_go<float, COLL_MRT>(g, p, s);
+  if (coll != COLL_BGK) return hipErrorInvalidValue;  // 16-bit storage: the host keeps MRT to single steps
+  return storage == 2 ? pair_go<_Float16, COLL_BGK>(g, p, s) : pair_go<bf16s, COLL_BGK>(g, p, s);
 }
 
 template <class S>

@@ -2,8 +2,8 @@
 
 HLBM_PAIRS=2 takes the two-step kernel at every size, HLBM_PAIRS=0 never.  The
 node's arithmetic is the same code, so every population must be equal bit for
-bit: FP64 against the oracle, the reduced storages (of which FP32 has the
-kernel) against single steps.  Sizes around the tile
+bit: FP64 against the oracle, the reduced storages (16-bit ones, BGK, rounding
+stochastically in between) against single steps.  Sizes around the tile
 (64 columns, 13 rows) and the segment, with rings that wrap onto the tile
 itself, faces on every axis and their edges and corners (the moving wall
 included), odd and even step counts, rho and u of the last step."""
