@@ -31,7 +31,7 @@ SYMBOLS = (
     "hlbm_last_error", "hlbm_version", "hlbm_device_count", "hlbm_domain_create", "hlbm_domain_destroy",
     "hlbm_domain_bytes", "hlbm_set_bcs", "hlbm_set_params", "hlbm_init_obst", "hlbm_add_obstacles",
     "hlbm_set_flags", "hlbm_get_flags", "hlbm_set_distribution", "hlbm_set_populations_f64",
-    "hlbm_get_populations_f64", "hlbm_step", "hlbm_timestep", "hlbm_synchronize", "hlbm_macro", "hlbm_get_macro",
+    "hlbm_get_populations_f64", "hlbm_step", "hlbm_steps_per_pass", "hlbm_timestep", "hlbm_synchronize", "hlbm_macro", "hlbm_get_macro",
     "hlbm_reduce_stats", "hlbm_ghost_update_ref", "hlbm_copy_bench", "hlbm_autotune", "hlbm_set_launch",
     "hlbm_set_collision", "hlbm_set_layout", "hlbm_get_layout", "hlbm_plane_profile", "hlbm_plane_profile_noalloc",
     "hlbm_line_velocity", "hlbm_init_double_couette",
@@ -154,6 +154,7 @@ def lib():
         "hlbm_set_populations_f64": (ctypes.c_int, [P, DP, ctypes.c_int32]),
         "hlbm_get_populations_f64": (ctypes.c_int, [P, DP, ctypes.c_int32]),
         "hlbm_step": (ctypes.c_int, [P, ctypes.c_int32, ctypes.c_uint32, P]),
+        "hlbm_steps_per_pass": (ctypes.c_int, [P, ctypes.POINTER(ctypes.c_int32)]),
         "hlbm_timestep": (ctypes.c_int, [P, ctypes.POINTER(ctypes.c_int64)]),
         "hlbm_synchronize": (ctypes.c_int, [P]),
         "hlbm_macro": (ctypes.c_int, [P, DP, DP, ctypes.c_int32]),

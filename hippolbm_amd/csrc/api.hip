@@ -89,6 +89,7 @@ struct hlbm_domain {
   int npt = 1;
   int force_wide = 0;
   int linear = 1;   // consecutive nodes per workgroup on ragged grids: 0 never, 1 large domains, 2 any size
+  bool pairs_tuned = true;  // false: the autotuner measured single steps faster
   int pairs = 1;    // two steps per pass where it applies: 0 never, 1 large domains, 2 any size
   int variant = 0;  // bulk-kernel variant (hlbm_set_launch)
   int boundary_first = 1;  // program-plane kernel before the bulk kernel (measured 1-2 % faster)
@@ -423,7 +424,7 @@ static int launch(hlbm_domain* h, int mode, bool write_macro, hipStream_t s, voi
 // Two steps in one pass (pair_kernel): domains whose every node runs the plain
 // pull, collide, store, and large enough to fill the chip with its tiles.
 static bool steps_in_pairs(const hlbm_domain* h, const StepParams& p, PairGrid* g) {
-  if (!h->pairs || h->d.pattern != HLBM_PATTERN_AB) return false;
+  if (!h->pairs || !h->pairs_tuned || h->d.pattern != HLBM_PATTERN_AB) return false;
   if (h->any_wall || p.nprog || p.prog_planes || p.nset || p.nspec || !default_layout_p(h)) return false;
   if (!p.pair32 || wide_offsets(p, h->esize)) return false;
   const bool narrow = h->esize == 2;
@@ -435,14 +436,17 @@ static bool steps_in_pairs(const hlbm_domain* h, const StepParams& p, PairGrid* 
   return h->pairs == 2 || (double)h->N >= fill * (double)cost * (PAIR_TX * PAIR_TY);
 }
 
-static int launch_pair(hlbm_domain* h, StepParams& p, PairGrid& g, bool write_macro, hipStream_t s) {
+static hipError_t run_pair(hlbm_domain* h, const StepParams& p, PairGrid g, hipStream_t s) {
+  const int coll = h->d.collision == HLBM_MRT ? COLL_MRT : COLL_BGK;
+  g.seed2 = step_seed(h->t + 1);
+  return h->d.storage == HLBM_F64 ? launch_pair_f64(coll, g, p, s) : launch_pair_lowp(h->d.storage, coll, g, p, s);
+}
+
+static int launch_pair(hlbm_domain* h, StepParams& p, const PairGrid& g, bool write_macro, hipStream_t s) {
   p.fin = h->buf[h->cur];
   p.fout = h->buf[h->cur ^ 1];
   p.write_macro = write_macro ? 1 : 0;
-  const int coll = h->d.collision == HLBM_MRT ? COLL_MRT : COLL_BGK;
-  g.seed2 = step_seed(h->t + 1);
-  const hipError_t e = h->d.storage == HLBM_F64 ? launch_pair_f64(coll, g, p, s)
-                                                : launch_pair_lowp(h->d.storage, coll, g, p, s);
+  const hipError_t e = run_pair(h, p, g, s);
   if (e != hipSuccess) return fail(HLBM_ERR_HIP, std::string("step pair launch: ") + hipGetErrorString(e));
   h->cur ^= 1;
   return HLBM_OK;
@@ -1132,6 +1136,13 @@ int hlbm_step(hlbm_domain* h, int32_t nsteps, uint32_t flags, void* stream) {
   return HLBM_OK;
 }
 
+int hlbm_steps_per_pass(hlbm_domain* h, int32_t* n) {
+  if (!h || !n) return fail(HLBM_ERR_ARG, "NULL argument");
+  PairGrid g;
+  *n = steps_in_pairs(h, base_params(h), &g) ? 2 : 1;
+  return HLBM_OK;
+}
+
 int hlbm_timestep(const hlbm_domain* h, int64_t* t) {
   if (!h || !t) return fail(HLBM_ERR_ARG, "NULL argument");
   *t = h->t;
@@ -1300,6 +1311,7 @@ int hlbm_set_launch(hlbm_domain* h, int32_t block_x, int32_t block_y, int32_t np
   if (variant != 0 && variant != 1) return fail(HLBM_ERR_ARG, "variant must be 0 or 1");
   h->block = dim3((unsigned)block_x, (unsigned)block_y, 1);
   h->variant = variant;
+  h->pairs_tuned = true;
   h->npt = variant == 1 ? 1 : npt;
   h->xcd_remap = xcd_remap ? 1 : 0;
   return HLBM_OK;
@@ -1361,14 +1373,16 @@ struct TuneVal {
   int bx, by, npt, remap, variant;
   double ms_best, ms_default;
   int order[3];
+  bool pairs;
 };
 std::mutex tune_mu;
 std::map<TuneKey, TuneVal> tune_cache;
 }  // namespace
 
-// Time `reps` steps with the domain's current launch shape on scratch memory.
+// Time `reps` steps with the domain's current launch shape on scratch memory; with
+// `pair`, passes of two steps (*ms is per step either way).
 static int time_shape(hlbm_domain* h, void* scratch, int reps, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
-                      double* ms) {
+                      double* ms, const PairGrid* pair = nullptr) {
   const bool aa = h->d.pattern == HLBM_PATTERN_AA;
   StepParams p = base_params(h);
   p.write_macro = 0;
@@ -1385,6 +1399,7 @@ static int time_shape(hlbm_domain* h, void* scratch, int reps, hipStream_t s, hi
       p.fin = h->buf[h->cur];
       p.fout = h->buf[h->cur ^ 1];  // overwritten by the next real step anyway
     }
+    if (pair) return run_pair(h, p, *pair, s);
     return run_kernels(h, p, mode, s);
   };
   hipError_t e = hipSuccess;
@@ -1396,7 +1411,7 @@ static int time_shape(hlbm_domain* h, void* scratch, int reps, hipStream_t s, hi
   float t = 0.f;
   if (e == hipSuccess) e = hipEventElapsedTime(&t, e0, e1);
   if (e != hipSuccess) return fail(HLBM_ERR_HIP, std::string("autotune: ") + hipGetErrorString(e));
-  *ms = (double)t / reps;
+  *ms = (double)t / reps / (pair ? 2 : 1);
   return HLBM_OK;
 }
 
@@ -1594,6 +1609,7 @@ int hlbm_autotune(hlbm_domain* h, int32_t reps, void* stream, hlbm_tune_info* ou
       const int rc = hlbm_set_layout(h, v.order);
       if (rc) return done(rc);
       hlbm_set_launch(h, v.bx, v.by, v.npt, v.remap, v.variant);
+      h->pairs_tuned = v.pairs;
       if (out)
         *out = hlbm_tune_info{v.bx, v.by, v.npt, v.remap, 0, v.variant, moved, pack_order(h), v.ms_best, v.ms_default};
       return done(HLBM_OK);
@@ -1615,7 +1631,7 @@ int hlbm_autotune(hlbm_domain* h, int32_t reps, void* stream, hlbm_tune_info* ou
   const dim3 keep_block = h->block;
   const int keep_npt = h->npt, keep_remap = h->xcd_remap, keep_variant = h->variant;
   static const int shapes[][2] = {{128, 2}, {64, 1}, {64, 2}, {64, 4}, {128, 1}, {256, 1}};
-  TuneVal best{128, 2, 1, 1, 0, 1e300, 0.0, {h->lay.ord[0], h->lay.ord[1], h->lay.ord[2]}};
+  TuneVal best{128, 2, 1, 1, 0, 1e300, 0.0, {h->lay.ord[0], h->lay.ord[1], h->lay.ord[2]}, true};
   int rc = HLBM_OK, n = 0;
   {
     // short steps: time enough of them that each candidate's measurement spans
@@ -1637,10 +1653,27 @@ int hlbm_autotune(hlbm_domain* h, int32_t reps, void* stream, hlbm_tune_info* ou
           if (sh[0] == 128 && sh[1] == 2 && npt == 1 && remap == 1 && variant == 0) best.ms_default = ms;
           if (ms < best.ms_best)
             best = TuneVal{sh[0], sh[1], npt, remap, variant, ms, best.ms_default, {best.order[0], best.order[1],
-                                                                                   best.order[2]}};
+                                                                                   best.order[2]}, true};
         }
       }
       if (rc) break;
+    }
+  }
+  // Two steps per pass, where they apply, against the best of the single steps:
+  // 16-bit storage is close (512^3 FP16 on tuned buffers 1.78-1.83 ms single,
+  // 1.84-1.87 in pairs; BF16 1.83-1.94, 1.73-1.75).  Taken, the domain keeps the
+  // 32-bit variant that they need.
+  if (rc == HLBM_OK) {
+    hlbm_set_launch(h, 128, 2, 1, 1, 0);
+    PairGrid g;
+    if (steps_in_pairs(h, base_params(h), &g)) {
+      double ms = 0.0;
+      rc = time_shape(h, scratch, reps, s, e0, e1, &ms, &g);
+      best.pairs = ms < best.ms_best;
+      if (best.pairs) {
+        if (best.variant) best.bx = 128, best.by = 2, best.npt = 1, best.remap = 1, best.variant = 0;
+        best.ms_best = ms;
+      }
     }
   }
   (void)hipEventDestroy(e0);
@@ -1654,6 +1687,7 @@ int hlbm_autotune(hlbm_domain* h, int32_t reps, void* stream, hlbm_tune_info* ou
     return rc;
   }
   hlbm_set_launch(h, best.bx, best.by, best.npt, best.remap, best.variant);
+  h->pairs_tuned = best.pairs;
   {
     std::lock_guard<std::mutex> g(tune_mu);
     tune_cache[key] = best;

@@ -188,6 +188,14 @@ class Domain:
         check("hlbm_timestep", lib().hlbm_timestep(self.h, ctypes.byref(t)))
         return t.value
 
+    @property
+    def steps_per_pass(self):
+        """Time steps `step` makes per read and write of the populations: 2 on large
+        A/B domains without walls and boundary programs, else 1."""
+        n = ctypes.c_int32(0)
+        check("hlbm_steps_per_pass", lib().hlbm_steps_per_pass(self.h, ctypes.byref(n)))
+        return n.value
+
     def autotune(self, reps=5, stream=None):
         """Pick the fastest node layout and launch shape for this domain (cached
         per shape); returns the choice and the per-step times."""

@@ -199,8 +199,13 @@ int hlbm_get_populations_f64(hlbm_domain* h, double* f, int32_t layout);
  * Advance nsteps reference time steps: macro_variables + collision +
  * pre_stream_bcs + streaming (+ update_ghost) + post_stream_bcs +
  * boundary_conditions (data/config/config_compute_loop.msp:28-36), fused into
- * one pull kernel per step.  Asynchronous on `stream`. */
+ * one pull kernel per step, or per two steps (hlbm_steps_per_pass; the results
+ * are the same bit for bit).  Asynchronous on `stream`. */
 int hlbm_step(hlbm_domain* h, int32_t nsteps, uint32_t flags, void* stream);
+/* *n = 2 if hlbm_step reads and writes the populations once per two steps (A/B
+ * domains without walls and boundary programs that fill the chip; an odd step of
+ * a call is made by itself), else 1. */
+int hlbm_steps_per_pass(hlbm_domain* h, int32_t* n);
 /* Steps taken since creation / the last set of populations. */
 int hlbm_timestep(const hlbm_domain* h, int64_t* t);
 int hlbm_synchronize(hlbm_domain* h);
