@@ -12,8 +12,9 @@ reported beside it under "per_dtype".
 
 Timing: HIP events on the stream the step kernels run on, W untimed warm-up
 steps, then exactly K timed steps, device synchronised before and after.
-Roofline: algorithmic bytes per node update = 2*19*sizeof(storage) + 1
-(flag byte) against MI355X's 8 TB/s HBM peak.
+Roofline: algorithmic bytes per node update = 2*19*sizeof(storage) / P + 1
+(flag byte) against MI355X's 8 TB/s HBM peak, where P is the time steps made
+per read and write of the populations (1 or 2, "steps_per_pass").
 """
 import argparse
 import json
@@ -65,15 +66,17 @@ def measure(n, storage, steps, warmup, collision="bgk", tune=True, pattern="ab")
     # sanity: the run stayed finite and mass-conserving
     dom.macro()
     st = dom.stats()
+    spp = dom.steps_per_pass
     dom.close()
     nodes = n ** 3
     ms_step = ms / steps
     mlups = nodes * steps / (ms * 1e-3) / 1e6
-    bpn = 2 * 19 * BYTES[storage] + 1
+    # a pass over the populations makes one step, or two: bytes of a node and step
+    bpn = 2 * 19 * BYTES[storage] / spp + 1
     gbs = nodes * bpn / (ms_step * 1e-3) / 1e9
-    return {"mlups": mlups, "ms_per_step": ms_step, "wall_s": wall, "bytes_per_node": bpn, "achieved_gbs": gbs,
-            "frac": gbs / HBM_PEAK_GBS, "sum_density": st["sum_density"], "max_u": st["max_velocity_norm"],
-            "launch": tuned}
+    return {"mlups": mlups, "ms_per_step": ms_step, "wall_s": wall, "bytes_per_node": bpn, "steps_per_pass": spp,
+            "achieved_gbs": gbs, "frac": gbs / HBM_PEAK_GBS, "sum_density": st["sum_density"],
+            "max_u": st["max_velocity_norm"], "launch": tuned}
 
 
 def porous_channel(steps=100, warmup=10, storage="f64", tune=True):
@@ -446,13 +449,15 @@ def main():
         "data": "synthetic (f_i = w_i, rho = 1)",
         "config": {"workload": f"couette_{n}^3_bgk_f64", "nodes": [n, n, n], "periodic": [True, True, False],
                    "tau": 0.8, "bcs": "pre_bounce_back + cavity_z_l(U=0.05) + post_bounce_back",
-                   "pattern": "AB pull, fused collide+stream"},
+                   "pattern": f"AB pull, fused collide+stream, {main_r['steps_per_pass']} steps per pass"},
         "roofline": {"bound": "hbm", "achieved": main_r["achieved_gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": main_r["frac"], "traffic": read_traffic(f"traffic_couette{n}_f64.txt"),
-                     "bytes_per_node": main_r["bytes_per_node"], "copy_kernel_gbs": copy_gbs,
+                     "bytes_per_node": main_r["bytes_per_node"], "steps_per_pass": main_r["steps_per_pass"],
+                     "copy_kernel_gbs": copy_gbs,
                      "launch": main_r["launch"]},
         "per_dtype": {k: {"mlups": v["mlups"], "frac": v["frac"], "achieved_gbs": v["achieved_gbs"],
-                          "bytes_per_node": v["bytes_per_node"], "ms_per_step": v["ms_per_step"]}
+                          "bytes_per_node": v["bytes_per_node"], "steps_per_pass": v["steps_per_pass"],
+                          "ms_per_step": v["ms_per_step"]}
                       for k, v in per.items()},
         "latency": ({"p50_s": served["f32"][0]["p50_s"], "p99_s": served["f32"][0]["p99_s"],
                      "requests": served["f32"][0]["n"], "failed": len(served["f32"][0]["failed"]),
