@@ -452,6 +452,14 @@ static int launch_pair(hlbm_domain* h, StepParams& p, const PairGrid& g, bool wr
   return HLBM_OK;
 }
 
+// A step graph that a caller captures is replayed on the buffers it was captured
+// with: an even number of single steps returns to the one it started from, a
+// single pass of two steps does not.
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return s && hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
 // Bring the state to the reference's post-stream/post-BC form f^T.
 static int materialize(hlbm_domain* h, hipStream_t s) {
   if (h->phase == PHASE_POST) {
@@ -1118,7 +1126,7 @@ int hlbm_step(hlbm_domain* h, int32_t nsteps, uint32_t flags, void* stream) {
       if (h->phase == PHASE_POST && k + 2 <= nsteps) {
         StepParams p = base_params(h);
         PairGrid g;
-        if (steps_in_pairs(h, p, &g)) {
+        if (steps_in_pairs(h, p, &g) && !capturing(s)) {
           const int rc = launch_pair(h, p, g, (flags & HLBM_STEP_WRITE_MACRO) && k + 2 == nsteps, s);
           if (rc) return rc;
           h->t += 2;

@@ -7,6 +7,8 @@ stochastically in between) against single steps.  Sizes around the tile
 (64 columns, 13 rows) and the segment, with rings that wrap onto the tile
 itself, faces on every axis and their edges and corners (the moving wall
 included), odd and even step counts, rho and u of the last step."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -101,3 +103,32 @@ def test_pairs_above_the_cache(n, monkeypatch):
         runs.append(sim.dom.get_f())
         sim.dom.close()
     assert np.array_equal(runs[0], runs[1])
+
+
+def test_captured_steps_replay(monkeypatch):
+    """A captured call of two steps advances by two steps on every replay: it
+    holds single steps, which return to the buffer they started from."""
+    from hippolbm_amd import hip
+    n = (70, 30, 20)
+    d = deck(n, (1, 0, 0), "bgk", 1e-4)
+    f0 = W.reshape(19, 1, 1, 1) * (1.0 + 1e-2 * np.random.default_rng(6).uniform(-1, 1, (19, n[2], n[1], n[0])))
+    sim = start(d, n, "f64", monkeypatch, 2, f0)
+    sim.run(3)
+    stream, h = hip.Stream(), hip.hip()
+    hip.device_synchronize()
+    graph, ex = ctypes.c_void_p(), ctypes.c_void_p()
+    assert h.hipStreamBeginCapture(stream.s, 2) == 0  # relaxed
+    sim.dom.step(2, stream=stream.handle)
+    assert h.hipStreamEndCapture(stream.s, ctypes.byref(graph)) == 0
+    assert h.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        assert h.hipGraphLaunch(ex, stream.s) == 0
+        stream.synchronize()
+    got = sim.dom.get_f()
+    h.hipGraphExecDestroy(ex)
+    h.hipGraphDestroy(graph)
+    stream.close()
+    sim.dom.close()
+    ref = orc.OracleRun(d, init_f=f0)
+    ref.step(9)
+    assert np.array_equal(got, ref.o.node_f())
