@@ -40,10 +40,10 @@ enum Phase { PHASE_PRE = 0, PHASE_POST = 1, PHASE_AA_PENDING = 2, PHASE_AA_SWAPP
 
 // The share of a two-step launch's lanes and planes that must be the domain's
 // own for it to be taken.  Single steps / pairs, us per step, BGK, couette:
-//   FP64  80^3 (0.34) 26 / 31   97^3 (0.48) 54 / 47   130^3 (0.54) 131 / 124
-//         112^3 (0.66) 86 / 66   256^3 (0.90) 983 / 660
-//   FP32  64^3 (0.31) 9.8 / 8.5   80^3 17.5 / 17.0   130^3 64 / 64   256^3 487 / 279
-//   16-bit (BGK, rows of whole half lines)  128^3 (0.76) 34 / 34   256^3 (0.90) 252 / 236
+//   FP64  64^3 (0.31) 14.8 / 17.2   63 x 80 x 80 (0.38) 21.6 / 22.5   97^3 (0.48) 53 / 45
+//         151 x 150 x 149 (0.66) 208 / 173   112^3 (0.66) 86 / 58
+//   FP32  64^3 9.5 / 8.1   63 x 80 x 80 14.8 / 10.4   151 x 150 x 149 104 / 96   112^3 41 / 31
+//   16-bit (BGK, rows of whole half lines)  128^3 (0.76) 34 / 34   256 x 200 x 100 (0.89) 84 / 74
 constexpr double PAIR_FILL_F64 = 0.45, PAIR_FILL_F32 = 0.3, PAIR_FILL_16 = 0.87;
 
 size_t elem_size(int storage) { return storage == HLBM_F64 ? 8 : (storage == HLBM_F32 ? 4 : 2); }

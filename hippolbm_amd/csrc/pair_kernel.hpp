@@ -44,7 +44,7 @@ namespace hlbm {
 constexpr int PAIR_TX = 64;  // tile columns along x: one wave per row
 // Tile rows: with the ring's two rows and the wave for its columns, the 16 waves
 // a workgroup can have.  The ring is stepped twice, so a step costs 16/13 of its
-// arithmetic (9 rows: 512^3 FP64 5.1-5.4 ms per step instead of 4.7).
+// arithmetic (9 rows: 512^3 FP64 5.1-5.4 ms per step where 13 took 4.7).
 constexpr int PAIR_TY = 13;
 
 struct PairGrid {

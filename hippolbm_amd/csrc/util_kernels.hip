@@ -361,7 +361,7 @@ __global__ void __launch_bounds__(RED_BLOCK)
 // The up to 1024 partials are latency-bound: one thread walking them alone made
 // a chain of dependent loads (20 us for the 117 partials of a 31^3 grid, about
 // 220 us for 1024); a block of 256 threads takes at most four records each and
-// then the same tree as the partial kernel: hlbm_reduce_stats 257 -> 27 us at
+// then the same tree as the partial kernel: hlbm_reduce_stats 257 -> 33 us at
 // 64^3, a step with its log line at 31^3 53 -> 28 us.
 __global__ void __launch_bounds__(RED_BLOCK) k_reduce_final(const double* part, int nparts, double* out) {
   double v[RED_VALUES];
