@@ -373,8 +373,10 @@ double hlbm_clock(void);
  * to a faster one (out->relocated; rejected buffers stay allocated until the
  * search ends so that each try lands elsewhere, so it uses up to four times the
  * population memory while free memory allows, keeping 4 GiB free;
- * HLBM_PLACEMENT=0 turns it off).  Results never depend on the
- * shape or the placement: every node runs the same arithmetic. */
+ * HLBM_PLACEMENT=0 turns it off).  Where hlbm_step can make two steps
+ * per pass (hlbm_steps_per_pass), that is timed too, beside the counted shapes,
+ * and kept or left.  Results never depend on the choice or the placement: every
+ * node runs the same arithmetic. */
 typedef struct {
   int32_t block_x, block_y, npt, xcd_remap; /* chosen shape */
   int32_t candidates;                       /* shapes timed; 0 = taken from the cache */
@@ -388,7 +390,8 @@ typedef struct {
 int hlbm_autotune(hlbm_domain* h, int32_t reps, void* stream, hlbm_tune_info* out);
 /* Set the shape by hand: block_x*block_y a multiple of 64 and <= 256, npt 1|2,
  * variant 0|1 (domains above 2^32 bytes per population plane, or with
- * start_iteration boxes, always take variant 1). */
+ * start_iteration boxes, always take variant 1).  Variant 1 makes one step per
+ * pass; variant 0 leaves two per pass to hlbm_step's own rule. */
 int hlbm_set_launch(hlbm_domain* h, int32_t block_x, int32_t block_y, int32_t npt, int32_t xcd_remap,
                     int32_t variant);
 
