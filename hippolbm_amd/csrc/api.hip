@@ -568,12 +568,12 @@ int hlbm_domain_create(const hlbm_domain_desc* desc, hlbm_domain** out) {
   if (hipMalloc((void**)&h->flags, N64) != hipSuccess) return cleanup("flags");
   if (hipMalloc((void**)&h->m0, N64 * 8) != hipSuccess) return cleanup("rho");
   if (hipMalloc((void**)&h->m1, N64 * 24) != hipSuccess) return cleanup("u");
-  if (hipMalloc((void**)&h->red_part, 7 * 8 * 1024) != hipSuccess) return cleanup("reduction");
-  if (hipMalloc((void**)&h->red_out, 7 * 8) != hipSuccess) return cleanup("reduction");
+  if (hipMalloc((void**)&h->red_part, RED_SCRATCH_BYTES) != hipSuccess) return cleanup("reduction");
+  if (hipMalloc((void**)&h->red_out, RED_VALUES * 8) != hipSuccess) return cleanup("reduction");
   const size_t gbytes = ghost_count(h->nx, h->ny, h->nz);
   if (any_periodic(h) && (hipMalloc((void**)&h->gflags, gbytes) != hipSuccess || hipMemset(h->gflags, 0, gbytes) != hipSuccess))
     return cleanup("ghost flags");
-  h->bytes = (aa ? 1 : 2) * fbytes + N64 * (1 + 8 + 24) + 7 * 8 * 1025 + (h->gflags ? gbytes : 0);
+  h->bytes = (aa ? 1 : 2) * fbytes + N64 * (1 + 8 + 24) + RED_SCRATCH_BYTES + RED_VALUES * 8 + (h->gflags ? gbytes : 0);
   if (hipMemset(h->buf[0], 0, fbytes) != hipSuccess || (!aa && hipMemset(h->buf[1], 0, fbytes) != hipSuccess) ||
       hipMemset(h->flags, 0, N64) != hipSuccess || hipMemset(h->m0, 0, N64 * 8) != hipSuccess ||
       hipMemset(h->m1, 0, N64 * 24) != hipSuccess)

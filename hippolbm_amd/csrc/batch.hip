@@ -385,8 +385,7 @@ int hlbm_batch_create(const hlbm_batch_desc* desc, hlbm_batch** out) {
   if (hipMalloc((void**)&b->d_doms, b->max_doms * sizeof(BatchDomain)) != hipSuccess) return cleanup("domains");
   if (hipMalloc((void**)&b->d_tiles, b->max_tiles * sizeof(BatchTile)) != hipSuccess) return cleanup("tiles");
   if (hipMalloc((void**)&b->d_ntiles, 2 * sizeof(uint32_t)) != hipSuccess) return cleanup("tile count");
-  if (hipMalloc((void**)&b->d_part, 7 * sizeof(double) * (size_t)reduce_parts(0xFFFFFFFFu)) != hipSuccess)
-    return cleanup("reduction partials");
+  if (hipMalloc((void**)&b->d_part, RED_SCRATCH_BYTES) != hipSuccess) return cleanup("reduction partials");
   for (int k = 0; k < 2; k++) {
     if (hipHostMalloc((void**)&b->h_doms_set[k], b->max_doms * sizeof(BatchDomain)) != hipSuccess ||
         hipHostMalloc((void**)&b->h_tiles_set[k], b->max_tiles * sizeof(BatchTile)) != hipSuccess ||

@@ -308,10 +308,7 @@ __global__ void k_macro(const void* fv, uint64_t stride, uint32_t N, const uint8
 // simulation_state (simulation_state.hpp:47-79): per-block partial sums in
 // FP64, then one block folds the partials, both in a fixed order
 // (deterministic).  Seven values per record: sum rho, min |u|, max |u|, the
-// three sums of rho u, the number of fluid nodes.
-constexpr int RED_BLOCK = 256;
-constexpr int RED_VALUES = 7;
-
+// three sums of rho u, the number of fluid nodes (sizes in reduce_parts.hpp).
 __device__ __forceinline__ double red_combine(int k, double a, double b) {
   return k == 1 ? fmin(a, b) : (k == 2 ? fmax(a, b) : a + b);
 }
@@ -746,11 +743,6 @@ hipError_t launch_placement_probe(const void* a, void* b, uint32_t n, hipStream_
   if (n == 0 || n % 256 != 0) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_placement_probe, dim3(n / 256), dim3(256), 0, s, (const uint16_t*)a, (uint16_t*)b, n);
   return hipGetLastError();
-}
-
-int reduce_parts(uint32_t N) {
-  int parts = (int)((N + RED_BLOCK - 1) / RED_BLOCK);
-  return parts > 1024 ? 1024 : (parts < 1 ? 1 : parts);
 }
 
 size_t profile_parts(int nx, int ny, int nz, int dim) { return (size_t)nx * (dim == 1 ? ny : nz); }
