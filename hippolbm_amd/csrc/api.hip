@@ -90,6 +90,7 @@ struct hlbm_domain {
   int force_wide = 0;
   int linear = 1;   // consecutive nodes per workgroup on ragged grids: 0 never, 1 large domains, 2 any size
   bool pairs_tuned = true;  // false: the autotuner measured single steps faster
+  bool captured = false;    // a step was captured: its graph may be replayed between live steps
   int pairs = 1;    // two steps per pass where it applies: 0 never, 1 large domains, 2 any size
   int variant = 0;  // bulk-kernel variant (hlbm_set_launch)
   int boundary_first = 1;  // program-plane kernel before the bulk kernel (measured 1-2 % faster)
@@ -424,7 +425,7 @@ static int launch(hlbm_domain* h, int mode, bool write_macro, hipStream_t s, voi
 // Two steps in one pass (pair_kernel): domains whose every node runs the plain
 // pull, collide, store, and large enough to fill the chip with its tiles.
 static bool steps_in_pairs(const hlbm_domain* h, const StepParams& p, PairGrid* g) {
-  if (!h->pairs || !h->pairs_tuned || h->d.pattern != HLBM_PATTERN_AB) return false;
+  if (!h->pairs || !h->pairs_tuned || h->captured || h->d.pattern != HLBM_PATTERN_AB) return false;
   if (h->any_wall || p.nprog || p.prog_planes || p.nset || p.nspec || !default_layout_p(h)) return false;
   if (!p.pair32 || wide_offsets(p, h->esize)) return false;
   const bool narrow = h->esize == 2;
@@ -454,7 +455,9 @@ static int launch_pair(hlbm_domain* h, StepParams& p, const PairGrid& g, bool wr
 
 // A step graph that a caller captures is replayed on the buffers it was captured
 // with: an even number of single steps returns to the one it started from, a
-// single pass of two steps does not.
+// single pass of two steps does not.  That holds for the live steps between two
+// replays as well, so a domain whose steps were captured once keeps to single
+// steps.
 static bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return s && hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
@@ -1113,6 +1116,7 @@ int hlbm_step(hlbm_domain* h, int32_t nsteps, uint32_t flags, void* stream) {
   if (!h || nsteps < 0) return fail(HLBM_ERR_ARG, "bad step arguments");
   hipStream_t s = (hipStream_t)stream;
   const bool aa = h->d.pattern == HLBM_PATTERN_AA;
+  if (nsteps > 0 && !h->captured && capturing(s)) h->captured = true;
   for (int k = 0; k < nsteps; k++) {
     const bool wm = (flags & HLBM_STEP_WRITE_MACRO) && k == nsteps - 1;
     if (aa) {
@@ -1126,7 +1130,7 @@ int hlbm_step(hlbm_domain* h, int32_t nsteps, uint32_t flags, void* stream) {
       if (h->phase == PHASE_POST && k + 2 <= nsteps) {
         StepParams p = base_params(h);
         PairGrid g;
-        if (steps_in_pairs(h, p, &g) && !capturing(s)) {
+        if (steps_in_pairs(h, p, &g)) {
           const int rc = launch_pair(h, p, g, (flags & HLBM_STEP_WRITE_MACRO) && k + 2 == nsteps, s);
           if (rc) return rc;
           h->t += 2;

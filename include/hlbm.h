@@ -200,11 +200,17 @@ int hlbm_get_populations_f64(hlbm_domain* h, double* f, int32_t layout);
  * pre_stream_bcs + streaming (+ update_ghost) + post_stream_bcs +
  * boundary_conditions (data/config/config_compute_loop.msp:28-36), fused into
  * one pull kernel per step, or per two steps (hlbm_steps_per_pass; the results
- * are the same bit for bit).  Asynchronous on `stream`. */
+ * are the same bit for bit).  Asynchronous on `stream`.
+ * A call may be captured into a graph.  A replay reads and writes the buffers of
+ * its capture, so it continues the current state if an even number of steps was
+ * captured, after at least one step, and every live call since then made an even
+ * number of steps (or read rho and u with hlbm_get_macro); an odd number, and
+ * calls that read or change populations, flags or operators, end that.  From the
+ * first captured call on the domain makes one step per pass. */
 int hlbm_step(hlbm_domain* h, int32_t nsteps, uint32_t flags, void* stream);
 /* *n = 2 if hlbm_step reads and writes the populations once per two steps (A/B
- * domains without walls and boundary programs that fill the chip; an odd step of
- * a call is made by itself), else 1. */
+ * domains without walls and boundary programs that fill the chip and whose steps
+ * were never captured; an odd step of a call is made by itself), else 1. */
 int hlbm_steps_per_pass(hlbm_domain* h, int32_t* n);
 /* Steps taken since creation / the last set of populations. */
 int hlbm_timestep(const hlbm_domain* h, int64_t* t);
