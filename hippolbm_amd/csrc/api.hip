@@ -92,6 +92,8 @@ struct hlbm_domain {
   bool pairs_tuned = true;  // false: the autotuner measured single steps faster
   bool captured = false;    // a step was captured: its graph may be replayed between live steps
   int pairs = 1;    // two steps per pass where it applies: 0 never, 1 large domains, 2 any size
+  PairGrid pair{};          // that launch (plan_pairs)
+  bool pair_fills = false;  // the domain fills the chip with it
   int variant = 0;  // bulk-kernel variant (hlbm_set_launch)
   int boundary_first = 1;  // program-plane kernel before the bulk kernel (measured 1-2 % faster)
   // the program-plane kernel on a second stream beside the bulk kernel
@@ -185,6 +187,11 @@ static RestShift dom_shift(const hlbm_domain* h) {
 // The rounding seed of time step t.
 static uint32_t step_seed(int64_t t) { return mix32((uint32_t)t * 0x9E3779B9u + 1u); }
 
+// 32-bit byte offsets reach both planes of a direction and its opposite.
+static bool plane_pairs_32bit(const hlbm_domain* h) {
+  return ((uint64_t)h->stride + h->N) * h->esize < 0xFFFFFFFFull;
+}
+
 static StepParams base_params(hlbm_domain* h) {
   StepParams p = h->plan;
   p.nx = h->nx;
@@ -231,7 +238,7 @@ static StepParams base_params(hlbm_domain* h) {
   p.spec_val = h->spec_val;
   p.force_wide = h->force_wide || h->variant == 1 ? 1 : 0;
   p.boundary_first = h->boundary_first;
-  p.pair32 = ((uint64_t)h->stride + h->N) * h->esize < 0xFFFFFFFFull ? 1 : 0;
+  p.pair32 = plane_pairs_32bit(h) ? 1 : 0;
   // 16-bit storage: stochastic rounding keyed on (node, time step)
   p.sr = (h->d.storage == HLBM_F16 || h->d.storage == HLBM_BF16) && !h->d.round_nearest ? 1 : 0;
   p.seed = step_seed(h->t);
@@ -424,30 +431,38 @@ static int launch(hlbm_domain* h, int mode, bool write_macro, hipStream_t s, voi
 
 // Two steps in one pass (pair_kernel): domains whose every node runs the plain
 // pull, collide, store, and large enough to fill the chip with its tiles.
-static bool steps_in_pairs(const hlbm_domain* h, const StepParams& p, PairGrid* g) {
+static bool steps_in_pairs(const hlbm_domain* h) {
   if (!h->pairs || !h->pairs_tuned || h->captured || h->d.pattern != HLBM_PATTERN_AB) return false;
-  if (h->any_wall || p.nprog || p.prog_planes || p.nset || p.nspec || !default_layout_p(h)) return false;
-  if (!p.pair32 || wide_offsets(p, h->esize)) return false;
-  const bool narrow = h->esize == 2;
-  if (narrow && h->d.collision == HLBM_MRT) return false;
-  const double fill = h->d.storage == HLBM_F64 ? PAIR_FILL_F64 : (narrow ? PAIR_FILL_16 : PAIR_FILL_F32);
-  int64_t cost;
-  *g = pair_grid(h->nx, h->ny, h->nz, &cost);
-  if (h->pairs == 1 && narrow && h->nx % 32 != 0) return false;
-  return h->pairs == 2 || (double)h->N >= fill * (double)cost * (PAIR_TX * PAIR_TY);
+  if (h->pairs == 1 && !h->pair_fills) return false;
+  const StepParams& p = h->plan;
+  if (h->any_wall || p.nprog || p.prog_planes || p.nset || !default_layout_p(h)) return false;
+  if (!plane_pairs_32bit(h) || h->force_wide || h->variant == 1) return false;
+  return !(h->esize == 2 && h->d.collision == HLBM_MRT);
 }
 
-static hipError_t run_pair(hlbm_domain* h, const StepParams& p, PairGrid g, hipStream_t s) {
+// The two-step launch of a domain's grid, and whether it fills the chip: both
+// depend on the grid and the storage only, so they are found once.
+static void plan_pairs(hlbm_domain* h) {
+  const bool narrow = h->esize == 2;
+  const double fill = h->d.storage == HLBM_F64 ? PAIR_FILL_F64 : (narrow ? PAIR_FILL_16 : PAIR_FILL_F32);
+  int64_t cost;
+  h->pair = pair_grid(h->nx, h->ny, h->nz, &cost);
+  h->pair_fills = (double)h->N >= fill * (double)cost * (PAIR_TX * PAIR_TY) && !(narrow && h->nx % 32 != 0);
+}
+
+static hipError_t run_pair(hlbm_domain* h, const StepParams& p, hipStream_t s) {
   const int coll = h->d.collision == HLBM_MRT ? COLL_MRT : COLL_BGK;
+  PairGrid g = h->pair;
   g.seed2 = step_seed(h->t + 1);
   return h->d.storage == HLBM_F64 ? launch_pair_f64(coll, g, p, s) : launch_pair_lowp(h->d.storage, coll, g, p, s);
 }
 
-static int launch_pair(hlbm_domain* h, StepParams& p, const PairGrid& g, bool write_macro, hipStream_t s) {
+static int launch_pair(hlbm_domain* h, bool write_macro, hipStream_t s) {
+  StepParams p = base_params(h);
   p.fin = h->buf[h->cur];
   p.fout = h->buf[h->cur ^ 1];
   p.write_macro = write_macro ? 1 : 0;
-  const hipError_t e = run_pair(h, p, g, s);
+  const hipError_t e = run_pair(h, p, s);
   if (e != hipSuccess) return fail(HLBM_ERR_HIP, std::string("step pair launch: ") + hipGetErrorString(e));
   h->cur ^= 1;
   return HLBM_OK;
@@ -557,6 +572,7 @@ int hlbm_domain_create(const hlbm_domain_desc* desc, hlbm_domain** out) {
     if (sscanf(blk, "%dx%d", &bx, &by) == 2 && bx > 0 && by > 0 && bx * by <= 256 && (bx * by) % 64 == 0)
       h->block = dim3(bx, by, 1);
   }
+  plan_pairs(h);
   const size_t fbytes = (size_t)h->stride * Q * h->esize;
   auto cleanup = [&](const std::string& what) {
     for (void* p : {h->buf[0], h->buf[1], (void*)h->flags, (void*)h->m0, (void*)h->m1, (void*)h->red_part,
@@ -1127,16 +1143,12 @@ int hlbm_step(hlbm_domain* h, int32_t nsteps, uint32_t flags, void* stream) {
       if (rc) return rc;
       h->phase = even ? PHASE_AA_SWAPPED : PHASE_AA_PENDING;
     } else {
-      if (h->phase == PHASE_POST && k + 2 <= nsteps) {
-        StepParams p = base_params(h);
-        PairGrid g;
-        if (steps_in_pairs(h, p, &g)) {
-          const int rc = launch_pair(h, p, g, (flags & HLBM_STEP_WRITE_MACRO) && k + 2 == nsteps, s);
-          if (rc) return rc;
-          h->t += 2;
-          k++;
-          continue;
-        }
+      if (h->phase == PHASE_POST && k + 2 <= nsteps && steps_in_pairs(h)) {
+        const int rc = launch_pair(h, (flags & HLBM_STEP_WRITE_MACRO) && k + 2 == nsteps, s);
+        if (rc) return rc;
+        h->t += 2;
+        k++;
+        continue;
       }
       const int mode = h->phase == PHASE_PRE ? MODE_COLLIDE : MODE_FUSED;
       int rc = launch(h, mode, wm, s);
@@ -1150,8 +1162,7 @@ int hlbm_step(hlbm_domain* h, int32_t nsteps, uint32_t flags, void* stream) {
 
 int hlbm_steps_per_pass(hlbm_domain* h, int32_t* n) {
   if (!h || !n) return fail(HLBM_ERR_ARG, "NULL argument");
-  PairGrid g;
-  *n = steps_in_pairs(h, base_params(h), &g) ? 2 : 1;
+  *n = steps_in_pairs(h) ? 2 : 1;
   return HLBM_OK;
 }
 
@@ -1394,7 +1405,7 @@ std::map<TuneKey, TuneVal> tune_cache;
 // Time `reps` steps with the domain's current launch shape on scratch memory; with
 // `pair`, passes of two steps (*ms is per step either way).
 static int time_shape(hlbm_domain* h, void* scratch, int reps, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
-                      double* ms, const PairGrid* pair = nullptr) {
+                      double* ms, bool pair = false) {
   const bool aa = h->d.pattern == HLBM_PATTERN_AA;
   StepParams p = base_params(h);
   p.write_macro = 0;
@@ -1411,7 +1422,7 @@ static int time_shape(hlbm_domain* h, void* scratch, int reps, hipStream_t s, hi
       p.fin = h->buf[h->cur];
       p.fout = h->buf[h->cur ^ 1];  // overwritten by the next real step anyway
     }
-    if (pair) return run_pair(h, p, *pair, s);
+    if (pair) return run_pair(h, p, s);
     return run_kernels(h, p, mode, s);
   };
   hipError_t e = hipSuccess;
@@ -1677,10 +1688,9 @@ int hlbm_autotune(hlbm_domain* h, int32_t reps, void* stream, hlbm_tune_info* ou
   // 32-bit variant that they need.
   if (rc == HLBM_OK) {
     hlbm_set_launch(h, 128, 2, 1, 1, 0);
-    PairGrid g;
-    if (steps_in_pairs(h, base_params(h), &g)) {
+    if (steps_in_pairs(h)) {
       double ms = 0.0;
-      rc = time_shape(h, scratch, reps, s, e0, e1, &ms, &g);
+      rc = time_shape(h, scratch, reps, s, e0, e1, &ms, true);
       best.pairs = ms < best.ms_best;
       if (best.pairs) {
         if (best.variant) best.bx = 128, best.by = 2, best.npt = 1, best.remap = 1, best.variant = 0;
