@@ -46,6 +46,10 @@ enum Phase { PHASE_PRE = 0, PHASE_POST = 1, PHASE_AA_PENDING = 2, PHASE_AA_SWAPP
 //   16-bit (BGK, rows of whole half lines)  128^3 (0.76) 34 / 34   256 x 200 x 100 (0.89) 84 / 74
 constexpr double PAIR_FILL_F64 = 0.45, PAIR_FILL_F32 = 0.3, PAIR_FILL_16 = 0.87;
 
+// Two steps per pass where they apply, unless the autotuner measured single steps
+// faster for this domain and collision or hlbm_set_launch asked for variant 1.
+enum PairChoice { PAIRS_BY_RULE = 0, PAIRS_SLOWER = 1, PAIRS_OFF_BY_HAND = 2 };
+
 size_t elem_size(int storage) { return storage == HLBM_F64 ? 8 : (storage == HLBM_F32 ? 4 : 2); }
 
 }  // namespace
@@ -89,7 +93,7 @@ struct hlbm_domain {
   int npt = 1;
   int force_wide = 0;
   int linear = 1;   // consecutive nodes per workgroup on ragged grids: 0 never, 1 large domains, 2 any size
-  bool pairs_tuned = true;  // false: the autotuner measured single steps faster
+  PairChoice pair_choice = PAIRS_BY_RULE;
   bool captured = false;    // a step was captured: its graph may be replayed between live steps
   int pairs = 1;    // two steps per pass where it applies: 0 never, 1 large domains, 2 any size
   PairGrid pair{};          // that launch (plan_pairs)
@@ -431,14 +435,15 @@ static int launch(hlbm_domain* h, int mode, bool write_macro, hipStream_t s, voi
 
 // Two steps in one pass (pair_kernel): domains whose every node runs the plain
 // pull, collide, store, and large enough to fill the chip with its tiles.
-static bool steps_in_pairs(const hlbm_domain* h) {
-  if (!h->pairs || !h->pairs_tuned || h->captured || h->d.pattern != HLBM_PATTERN_AB) return false;
+static bool pairs_apply(const hlbm_domain* h) {
+  if (!h->pairs || h->captured || h->d.pattern != HLBM_PATTERN_AB) return false;
   if (h->pairs == 1 && !h->pair_fills) return false;
   const StepParams& p = h->plan;
   if (h->any_wall || p.nprog || p.prog_planes || p.nset || !default_layout_p(h)) return false;
-  if (!plane_pairs_32bit(h) || h->force_wide || h->variant == 1) return false;
+  if (!plane_pairs_32bit(h) || h->force_wide) return false;
   return !(h->esize == 2 && h->d.collision == HLBM_MRT);
 }
+static bool steps_in_pairs(const hlbm_domain* h) { return h->pair_choice == PAIRS_BY_RULE && pairs_apply(h); }
 
 // The two-step launch of a domain's grid, and whether it fills the chip: both
 // depend on the grid and the storage only, so they are found once.
@@ -1309,6 +1314,7 @@ int hlbm_set_collision(hlbm_domain* h, int32_t collision, const double* mrt_rate
   }
   const RestShift old = dom_shift(h);
   h->d.collision = collision;
+  if (h->pair_choice == PAIRS_SLOWER) h->pair_choice = PAIRS_BY_RULE;  // measured with the old one
   h->d.mrt_custom = mrt_rates ? 1 : 0;
   for (int k = 0; k < 10; k++) h->d.mrt_rates[k] = mrt_rates ? mrt_rates[k] : 0.0;
   const RestShift now = dom_shift(h);
@@ -1325,6 +1331,15 @@ int hlbm_set_collision(hlbm_domain* h, int32_t collision, const double* mrt_rate
   return HLBM_OK;
 }
 
+// The launch shape alone: what the autotuner tries must not touch the choice of
+// steps per pass, which it would then have to put back.
+static void set_shape(hlbm_domain* h, int bx, int by, int npt, int remap, int variant) {
+  h->block = dim3((unsigned)bx, (unsigned)by, 1);
+  h->variant = variant;
+  h->npt = variant == 1 ? 1 : npt;
+  h->xcd_remap = remap ? 1 : 0;
+}
+
 int hlbm_set_launch(hlbm_domain* h, int32_t block_x, int32_t block_y, int32_t npt, int32_t xcd_remap,
                     int32_t variant) {
   if (!h) return fail(HLBM_ERR_ARG, "NULL domain");
@@ -1332,11 +1347,8 @@ int hlbm_set_launch(hlbm_domain* h, int32_t block_x, int32_t block_y, int32_t np
     return fail(HLBM_ERR_ARG, "block_x*block_y must be a multiple of 64 and at most 256");
   if (npt != 1 && npt != 2) return fail(HLBM_ERR_ARG, "npt must be 1 or 2");
   if (variant != 0 && variant != 1) return fail(HLBM_ERR_ARG, "variant must be 0 or 1");
-  h->block = dim3((unsigned)block_x, (unsigned)block_y, 1);
-  h->variant = variant;
-  h->pairs_tuned = true;
-  h->npt = variant == 1 ? 1 : npt;
-  h->xcd_remap = xcd_remap ? 1 : 0;
+  set_shape(h, block_x, block_y, npt, xcd_remap, variant);
+  h->pair_choice = variant == 1 ? PAIRS_OFF_BY_HAND : PAIRS_BY_RULE;
   return HLBM_OK;
 }
 
@@ -1384,19 +1396,22 @@ int hlbm_get_layout(const hlbm_domain* h, int32_t order[3]) {
 }
 
 namespace {
+// What the choice depends on: the grid and the kernels that its steps run.
+// walls: none, walls that block the two-step kernel only, walls with the mask.
+// order: the node layout, where it is given and not tuned (-1: program planes).
+// pairs: two steps per pass apply, so they were timed.
 struct TuneKey {
-  int nx, ny, nz, storage, collision, pattern, prog_planes, wall_bb, device;
-  bool operator<(const TuneKey& o) const {
-    const int a[9] = {nx, ny, nz, storage, collision, pattern, prog_planes, wall_bb, device};
-    const int b[9] = {o.nx, o.ny, o.nz, o.storage, o.collision, o.pattern, o.prog_planes, o.wall_bb, o.device};
-    return std::lexicographical_compare(a, a + 9, b, b + 9);
+  int nx, ny, nz, storage, collision, pattern, prog_planes, walls, boxes, order, pairs, linear, force_wide, device;
+  std::array<int, 14> all() const {
+    return {nx, ny, nz, storage, collision, pattern, prog_planes, walls, boxes, order, pairs, linear, force_wide, device};
   }
+  bool operator<(const TuneKey& o) const { return all() < o.all(); }
 };
 struct TuneVal {
   int bx, by, npt, remap, variant;
   double ms_best, ms_default;
   int order[3];
-  bool pairs;
+  bool pairs_slower;  // measured, where they apply
 };
 std::mutex tune_mu;
 std::map<TuneKey, TuneVal> tune_cache;
@@ -1555,7 +1570,7 @@ static int choose_layout(hlbm_domain* h, int reps, hipStream_t s, hipEvent_t e0,
   if (cand.size() < 2) return HLBM_OK;
   const dim3 keep_block = h->block;
   const int keep_npt = h->npt, keep_remap = h->xcd_remap, keep_variant = h->variant;
-  hlbm_set_launch(h, 128, 2, 1, 1, 0);
+  set_shape(h, 128, 2, 1, 1, 0);
   const bool aa = h->d.pattern == HLBM_PATTERN_AA;
   const size_t fbytes = (size_t)h->stride * Q * h->esize;
   double best = 1e300;
@@ -1623,7 +1638,9 @@ int hlbm_autotune(hlbm_domain* h, int32_t reps, void* stream, hlbm_tune_info* ou
     }
   }
   const TuneKey key{h->nx, h->ny, h->nz, h->d.storage, h->d.collision, h->d.pattern, h->plan.prog_planes,
-                    h->any_wall && h->plan.wall_bb ? 1 : 0, h->device};
+                    h->any_wall ? (h->plan.wall_bb ? 2 : 1) : 0, h->plan.nset ? 1 : 0,
+                    h->plan.prog_planes ? -1 : pack_order(h), pairs_apply(h) ? 1 : 0, h->linear, h->force_wide,
+                    h->device};
   {
     std::lock_guard<std::mutex> g(tune_mu);
     auto it = tune_cache.find(key);
@@ -1631,8 +1648,8 @@ int hlbm_autotune(hlbm_domain* h, int32_t reps, void* stream, hlbm_tune_info* ou
       const TuneVal v = it->second;
       const int rc = hlbm_set_layout(h, v.order);
       if (rc) return done(rc);
-      hlbm_set_launch(h, v.bx, v.by, v.npt, v.remap, v.variant);
-      h->pairs_tuned = v.pairs;
+      set_shape(h, v.bx, v.by, v.npt, v.remap, v.variant);
+      h->pair_choice = v.pairs_slower ? PAIRS_SLOWER : PAIRS_BY_RULE;
       if (out)
         *out = hlbm_tune_info{v.bx, v.by, v.npt, v.remap, 0, v.variant, moved, pack_order(h), v.ms_best, v.ms_default};
       return done(HLBM_OK);
@@ -1654,7 +1671,7 @@ int hlbm_autotune(hlbm_domain* h, int32_t reps, void* stream, hlbm_tune_info* ou
   const dim3 keep_block = h->block;
   const int keep_npt = h->npt, keep_remap = h->xcd_remap, keep_variant = h->variant;
   static const int shapes[][2] = {{128, 2}, {64, 1}, {64, 2}, {64, 4}, {128, 1}, {256, 1}};
-  TuneVal best{128, 2, 1, 1, 0, 1e300, 0.0, {h->lay.ord[0], h->lay.ord[1], h->lay.ord[2]}, true};
+  TuneVal best{128, 2, 1, 1, 0, 1e300, 0.0, {h->lay.ord[0], h->lay.ord[1], h->lay.ord[2]}, false};
   int rc = HLBM_OK, n = 0;
   {
     // short steps: time enough of them that each candidate's measurement spans
@@ -1668,7 +1685,7 @@ int hlbm_autotune(hlbm_domain* h, int32_t reps, void* stream, hlbm_tune_info* ou
       // a layout other than the default runs one node per thread
       for (int npt = 1; npt <= (variant || !default_layout_p(h) ? 1 : 2) && rc == HLBM_OK; npt++) {
         for (int remap = 1; remap >= 0 && rc == HLBM_OK; remap--) {
-          hlbm_set_launch(h, sh[0], sh[1], npt, remap, variant);
+          set_shape(h, sh[0], sh[1], npt, remap, variant);
           double ms = 0.0;
           rc = time_shape(h, scratch, reps, s, e0, e1, &ms);
           if (rc) break;
@@ -1676,7 +1693,7 @@ int hlbm_autotune(hlbm_domain* h, int32_t reps, void* stream, hlbm_tune_info* ou
           if (sh[0] == 128 && sh[1] == 2 && npt == 1 && remap == 1 && variant == 0) best.ms_default = ms;
           if (ms < best.ms_best)
             best = TuneVal{sh[0], sh[1], npt, remap, variant, ms, best.ms_default, {best.order[0], best.order[1],
-                                                                                   best.order[2]}, true};
+                                                                                   best.order[2]}, false};
         }
       }
       if (rc) break;
@@ -1684,19 +1701,13 @@ int hlbm_autotune(hlbm_domain* h, int32_t reps, void* stream, hlbm_tune_info* ou
   }
   // Two steps per pass, where they apply, against the best of the single steps:
   // 16-bit storage is close (512^3 FP16 on tuned buffers 1.78-1.83 ms single,
-  // 1.84-1.87 in pairs; BF16 1.83-1.94, 1.73-1.75).  Taken, the domain keeps the
-  // 32-bit variant that they need.
-  if (rc == HLBM_OK) {
-    hlbm_set_launch(h, 128, 2, 1, 1, 0);
-    if (steps_in_pairs(h)) {
-      double ms = 0.0;
-      rc = time_shape(h, scratch, reps, s, e0, e1, &ms, true);
-      best.pairs = ms < best.ms_best;
-      if (best.pairs) {
-        if (best.variant) best.bx = 128, best.by = 2, best.npt = 1, best.remap = 1, best.variant = 0;
-        best.ms_best = ms;
-      }
-    }
+  // 1.84-1.87 in pairs; BF16 1.83-1.94, 1.73-1.75).  The best single-step shape
+  // stays with the domain for the steps that are made alone.
+  if (rc == HLBM_OK && pairs_apply(h)) {
+    double ms = 0.0;
+    rc = time_shape(h, scratch, reps, s, e0, e1, &ms, true);
+    best.pairs_slower = !(ms < best.ms_best);
+    if (!best.pairs_slower) best.ms_best = ms;
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
@@ -1708,8 +1719,8 @@ int hlbm_autotune(hlbm_domain* h, int32_t reps, void* stream, hlbm_tune_info* ou
     h->variant = keep_variant;
     return rc;
   }
-  hlbm_set_launch(h, best.bx, best.by, best.npt, best.remap, best.variant);
-  h->pairs_tuned = best.pairs;
+  set_shape(h, best.bx, best.by, best.npt, best.remap, best.variant);
+  h->pair_choice = best.pairs_slower ? PAIRS_SLOWER : PAIRS_BY_RULE;
   {
     std::lock_guard<std::mutex> g(tune_mu);
     tune_cache[key] = best;

@@ -369,8 +369,9 @@ double hlbm_clock(void);
  * populations, phase and step count are left as they were: A/B domains write
  * only the buffer the next step overwrites; AA domains work on a temporary
  * copy), keeps the fastest for this domain and caches it per (dims, storage,
- * collision, pattern, boundary program, device) so later domains of the same
- * shape skip the search (out->candidates == 0).  Each candidate is timed over
+ * collision, pattern, boundary program, walls, start_iteration boxes, layout set
+ * by hand, whether two steps per pass apply, device) so later domains of the same
+ * kind skip the search (out->candidates == 0).  Each candidate is timed over
  * `reps` steps, or over as many as take about 5 ms when `reps` steps of the
  * default shape take less (at most 500).  First, a domain with 256 MiB
  * of populations or more checks its placement: the step speed
