@@ -630,7 +630,7 @@ int hlbm_domain_destroy(hlbm_domain* h) {
   if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
   if (h->ev_join) (void)hipEventDestroy(h->ev_join);
   if (h->side) (void)hipStreamDestroy(h->side);
-  free_ring(h->ring);
+  return_ring(h->ring, h->device);
   delete h;
   return HLBM_OK;
 }

@@ -10,9 +10,10 @@
 // order at the link's rate (53 GB/s to the host, 55 from it; conversion and
 // layout cost nothing there), and a few threads move it between the slots and
 // the caller's array, both sides running ahead of each other by half a ring.
-// The ring stays with the domain: the first touch of pinned memory costs 0.4 ms
-// a MiB, and a ring made anew by each call paid it in every other one.  Slots of
-// 512 KiB leave the link at 47 GB/s, 1 MiB (for 64 MiB and more) at 50.
+// The ring stays with the domain, and then for the next one: the first touch of
+// pinned memory costs up to 0.4 ms a MiB, and a ring made anew by each call paid it
+// in every other one.  Slots of 512 KiB leave the link at 47 GB/s, 1 MiB (for 64
+// MiB and more) at 50.
 // Measured against copies plane by plane through the runtime: 400 steps of the
 // porous channel 256 x 128 x 128 (layout "yzx") with rho and u read 215 -> 105
 // ms, 300 MRT steps of 128^3 FP32 35.5 -> 20.2 ms, populations of 96^3 in and
@@ -23,6 +24,7 @@
 #include <condition_variable>
 #include <cstring>
 #include <functional>
+#include <map>
 #include <mutex>
 #include <new>
 #include <system_error>
@@ -34,35 +36,106 @@
 
 namespace hlbm {
 
-constexpr size_t SLOT_SMALL = (size_t)512 << 10, SLOT_LARGE = (size_t)1 << 20, LARGE_FROM = (size_t)64 << 20;
+constexpr size_t MIB = (size_t)1 << 20;
+constexpr size_t SLOT_SMALL = MIB / 2, SLOT_LARGE = MIB, LARGE_FROM = 64 * MIB;
 constexpr int SLOTS = 16, THREADS = 8;
+constexpr size_t BLOCK = SLOTS * SLOT_SMALL;  // one pinned allocation: the small slots, or half of the large ones
+constexpr int BLOCKS = 2;
+static_assert(BLOCKS * BLOCK == SLOTS * SLOT_LARGE, "large slots fill all blocks");
 
 struct TransferRing {
-  double* mem = nullptr;
-  size_t slot_bytes = 0;
+  char* block[BLOCKS] = {};
   hipEvent_t ev[SLOTS] = {};
-  explicit TransferRing(size_t bytes) : slot_bytes(bytes) {}
+  int device = 0;
+  bool sound = true;  // no transfer through it has failed
   ~TransferRing() {
     for (hipEvent_t e : ev)
       if (e) (void)hipEventDestroy(e);
-    if (mem) (void)hipHostFree(mem);
+    for (char* b : block)
+      if (b) (void)hipHostFree(b);
   }
   bool open() {
-    if (hipHostMalloc((void**)&mem, slot_bytes * SLOTS, hipHostMallocCoherent) != hipSuccess) {
-      mem = nullptr;
-      (void)hipGetLastError();
-      return false;
-    }
+    if (hipGetDevice(&device) != hipSuccess || !pin(0)) return false;
     for (int k = 0; k < SLOTS; k++)
       if (hipEventCreateWithFlags(&ev[k], hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
         ev[k] = nullptr;
+        (void)hipGetLastError();
         return false;
       }
     return true;
   }
+  // Large slots need the second block, which is pinned beside the first by the
+  // first transfer that asks for them; without it the small ones serve on.
+  size_t slot_bytes(bool large) { return large && pin(1) ? SLOT_LARGE : SLOT_SMALL; }
+  double* slot(int k, size_t bytes) const {
+    const size_t per = BLOCK / bytes, i = (size_t)(k % SLOTS);
+    return (double*)(block[i / per] + i % per * bytes);
+  }
+
+ private:
+  bool pin(int b) {
+    if (!block[b] && hipHostMalloc((void**)&block[b], BLOCK, hipHostMallocCoherent) != hipSuccess) {
+      block[b] = nullptr;
+      (void)hipGetLastError();
+    }
+    return block[b] != nullptr;
+  }
 };
 
-void free_ring(TransferRing* ring) { delete ring; }
+// One ring per device waits for the next domain after its own was destroyed:
+// its pinned pages cost 1 to 2 ms, which a program that makes a domain, reads it
+// once and makes the next would pay each time (first read of new 44^3 FP64
+// domains, populations 1.7 ms against 0.8 ms later).  At most 16 MiB a device,
+// given back when SPARE_IDLE domains in a row have gone without large transfers.
+constexpr int SPARE_IDLE = 8;
+struct Spare {
+  TransferRing* ring = nullptr;
+  int idle = 0;
+};
+struct Spares {
+  std::mutex mu;
+  std::map<int, Spare> of;  // device -> spare
+};
+static Spares& spares() {
+  static Spares* s = new Spares;  // never destroyed: the runtime may be gone by then
+  return *s;
+}
+
+static TransferRing* take_ring() {
+  int device = 0;
+  if (hipGetDevice(&device) == hipSuccess) {
+    std::lock_guard<std::mutex> l(spares().mu);
+    const auto it = spares().of.find(device);
+    if (it != spares().of.end() && it->second.ring) {
+      TransferRing* r = it->second.ring;
+      it->second = Spare{};
+      return r;
+    }
+  }
+  TransferRing* r = new TransferRing;
+  if (r->open()) return r;
+  delete r;
+  return nullptr;
+}
+
+void return_ring(TransferRing* ring, int device) {
+  TransferRing* drop = nullptr;
+  try {
+    std::lock_guard<std::mutex> l(spares().mu);
+    Spare& s = spares().of[ring ? ring->device : device];
+    if (ring && ring->sound && !s.ring) {
+      s = Spare{ring, 0};
+    } else if (ring) {
+      drop = ring;
+    } else if (s.ring && ++s.idle >= SPARE_IDLE) {
+      drop = s.ring;
+      s = Spare{};
+    }
+  } catch (const std::bad_alloc&) {
+    drop = ring;
+  }
+  delete drop;
+}
 
 namespace {
 
@@ -70,7 +143,7 @@ namespace {
 // host 10 MiB 0.67 ms and 0.70 through the ring, 25 MiB 2.0 and 1.4; from warm
 // host pages 25 MiB 1.3 either way, 38 MiB 1.9 and 1.6), unless every plane has
 // to be rearranged on the host.
-constexpr size_t MIN_TO_HOST = (size_t)12 << 20, MIN_TO_DEVICE = (size_t)32 << 20, MIN_REARRANGED = (size_t)4 << 20;
+constexpr size_t MIN_TO_HOST = 12 * MIB, MIN_TO_DEVICE = 32 * MIB, MIN_REARRANGED = 4 * MIB;
 
 // node k of the host's order (x fastest) -> index in the device layout
 struct NodeOrder {
@@ -229,20 +302,11 @@ int transfer(TransferRing** owned, bool out, const TransferGrid& g, const NodePl
   const size_t total = (size_t)N * 8 * count;
   const bool perm = !(g.lay.ord[0] == 0 && g.lay.ord[1] == 1);
   if (total < (perm || g.reference ? MIN_REARRANGED : out ? MIN_TO_HOST : MIN_TO_DEVICE)) return TRANSFER_DECLINED;
-  if (*owned && total >= LARGE_FROM && (*owned)->slot_bytes < SLOT_LARGE) {
-    delete *owned;
-    *owned = nullptr;
-  }
-  if (!*owned) {
-    *owned = new TransferRing(total >= LARGE_FROM ? SLOT_LARGE : SLOT_SMALL);
-    if (!(*owned)->open()) {
-      delete *owned;
-      *owned = nullptr;
-      return TRANSFER_DECLINED;
-    }
-  }
+  if (!*owned) *owned = take_ring();
+  if (!*owned) return TRANSFER_DECLINED;
   TransferRing& ring = **owned;
-  const uint32_t per = (uint32_t)(ring.slot_bytes / 8);
+  const size_t slot_bytes = ring.slot_bytes(total >= LARGE_FROM);
+  const uint32_t per = (uint32_t)(slot_bytes / 8);
   constexpr int slots = SLOTS, ahead = SLOTS / 2;
   std::vector<Chunk> chunks;
   for (int p = 0; p < count; p++)
@@ -256,7 +320,7 @@ int transfer(TransferRing** owned, bool out, const TransferGrid& g, const NodePl
   node_divisor(o.nxy, o.div.m01, o.div.s01);
   o.lay = g.lay;
 
-  auto slot = [&](int c) { return ring.mem + (size_t)(c % slots) * per; };
+  auto slot = [&](int c) { return ring.slot(c, slot_bytes); };
   Copiers copiers(nc, [&](int c) {
     const Chunk& k = chunks[c];
     copy_rows(g, out, slot(c), planes[k.plane].host, k.first, k.n);
@@ -312,6 +376,7 @@ int transfer(TransferRing** owned, bool out, const TransferGrid& g, const NodePl
   // nothing may still read or write the slots afterwards
   const hipError_t last = hipStreamSynchronize(s);
   *err = e != hipSuccess ? e : last;
+  ring.sound = ring.sound && *err == hipSuccess;
   return *err == hipSuccess ? TRANSFER_DONE : TRANSFER_FAILED;
 }
 

@@ -30,10 +30,12 @@ struct TransferGrid {
   RestShift shift;
 };
 
-// The pinned slots of a domain's transfers: made by its first large one, kept
-// until the domain is destroyed (8 MiB, 16 MiB for 64 MiB and more).
+// The pinned slots of a domain's transfers: had by its first large one (8 MiB, 16
+// MiB from the first of 64 MiB and more), its own until it is destroyed.  Every
+// destroyed domain calls return_ring, with its ring or nullptr: one ring per
+// device waits there for the next domain.
 struct TransferRing;
-void free_ring(TransferRing* ring);
+void return_ring(TransferRing* ring, int device);
 
 enum TransferStatus { TRANSFER_DONE = 0, TRANSFER_DECLINED = 1, TRANSFER_FAILED = 2 };
 
