@@ -142,8 +142,12 @@ namespace {
 // Below these sizes the runtime's own copies of whole planes are as fast (to the
 // host 10 MiB 0.67 ms and 0.70 through the ring, 25 MiB 2.0 and 1.4; from warm
 // host pages 25 MiB 1.3 either way, 38 MiB 1.9 and 1.6), unless every plane has
-// to be rearranged on the host.
-constexpr size_t MIN_TO_HOST = 12 * MIB, MIN_TO_DEVICE = 32 * MIB, MIN_REARRANGED = 4 * MIB;
+// to be rearranged on the host.  Populations read in the reference layout pay a
+// little later than other rearranged planes: their rows are short copies for
+// either (4.3 MiB 0.54 and 0.60-0.74, 6.8 MiB 0.73 and 0.67-0.79, 33 MiB 5.8 and
+// 3.2).
+constexpr size_t MIN_TO_HOST = 12 * MIB, MIN_TO_DEVICE = 32 * MIB;
+constexpr size_t MIN_REARRANGED = 4 * MIB, MIN_REFERENCE_TO_HOST = 6 * MIB;
 
 // node k of the host's order (x fastest) -> index in the device layout
 struct NodeOrder {
@@ -301,7 +305,10 @@ int transfer(TransferRing** owned, bool out, const TransferGrid& g, const NodePl
   const uint32_t N = (uint32_t)g.n[0] * (uint32_t)g.n[1] * (uint32_t)g.n[2];
   const size_t total = (size_t)N * 8 * count;
   const bool perm = !(g.lay.ord[0] == 0 && g.lay.ord[1] == 1);
-  if (total < (perm || g.reference ? MIN_REARRANGED : out ? MIN_TO_HOST : MIN_TO_DEVICE)) return TRANSFER_DECLINED;
+  const bool populations = planes[0].q >= 0;
+  const size_t least = perm || g.reference ? (out && populations && !perm ? MIN_REFERENCE_TO_HOST : MIN_REARRANGED)
+                                           : (out ? MIN_TO_HOST : MIN_TO_DEVICE);
+  if (total < least) return TRANSFER_DECLINED;
   if (!*owned) *owned = take_ring();
   if (!*owned) return TRANSFER_DECLINED;
   TransferRing& ring = **owned;

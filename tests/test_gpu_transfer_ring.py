@@ -2,7 +2,8 @@
 first transfer of 64 MiB, one that passes from a destroyed domain to the next
 (other sizes, storages and layouts), several at once, each domain on a thread of
 its own, and one given back after enough domains without large transfers.  Exact,
-like the single transfers."""
+like the single transfers; and round trips at the sizes from which populations in
+the reference layout take the ring to the host."""
 import threading
 
 import numpy as np
@@ -12,6 +13,7 @@ from hippolbm_amd import _lib
 from hippolbm_amd.engine import W, Domain
 
 from test_gpu_transfer import stored
+from test_gpu_transfer import test_host_arrays_round_trip as round_trip
 
 pytestmark = pytest.mark.gpu
 
@@ -40,6 +42,14 @@ def check(dom, n, storage, seed, layout=_lib.LAYOUT_NODES):
         for i in range(19):
             rho += f[i]
         assert np.array_equal(dom.macro()[0], rho)
+
+
+# 19 x 34^3 and 35^3 doubles: either side of 6 MiB
+@pytest.mark.parametrize("n", [(34, 34, 34), (35, 35, 35)], ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("storage", ["f64", "f32", "f16", "bf16"])
+@pytest.mark.parametrize("order", [(0, 1, 2), (1, 2, 0)], ids=["xyz", "yzx"])
+def test_sizes_from_which_the_reference_layout_takes_the_ring(n, storage, order):
+    round_trip(n, storage, order)
 
 
 def test_a_ring_grows_and_serves_small_transfers_again():
