@@ -67,6 +67,17 @@ struct TransferRing {
   // Large slots need the second block, which is pinned beside the first by the
   // first transfer that asks for them; without it the small ones serve on.
   size_t slot_bytes(bool large) { return large && pin(1) ? SLOT_LARGE : SLOT_SMALL; }
+  // false after a reset of the device, which takes pinned memory with it
+  bool alive() const {
+    for (char* b : block) {
+      hipPointerAttribute_t a;
+      if (b && (hipPointerGetAttributes(&a, b) != hipSuccess || a.type != hipMemoryTypeHost)) {
+        (void)hipGetLastError();
+        return false;
+      }
+    }
+    return true;
+  }
   double* slot(int k, size_t bytes) const {
     const size_t per = BLOCK / bytes, i = (size_t)(k % SLOTS);
     return (double*)(block[i / per] + i % per * bytes);
@@ -109,7 +120,7 @@ static TransferRing* take_ring() {
     if (it != spares().of.end() && it->second.ring) {
       TransferRing* r = it->second.ring;
       it->second = Spare{};
-      return r;
+      if (r->alive()) return r;  // (else nothing of it is left to free)
     }
   }
   TransferRing* r = new TransferRing;
