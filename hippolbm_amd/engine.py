@@ -191,7 +191,8 @@ class Domain:
     @property
     def steps_per_pass(self):
         """Time steps `step` makes per read and write of the populations: 2 on large
-        A/B domains without walls and boundary programs, else 1."""
+        A/B domains without walls and boundary programs whose steps were never
+        captured into a graph, else 1."""
         n = ctypes.c_int32(0)
         check("hlbm_steps_per_pass", lib().hlbm_steps_per_pass(self.h, ctypes.byref(n)))
         return n.value
